@@ -12,10 +12,17 @@
 //   2. colptr = exclusive scan of the counts (three launches: block scans,
 //      the scan of the block totals, the offsets);
 //   3. every stored entry placed in its column's list (integer atomics on a
-//      cursor copied from colptr), then each list sorted by CSRC position, so
-//      the order, and the FP64 result, never depend on the atomics;
-//   4. the gather product: y_i = ad_i x_i + row i in CSRC order + column i in
-//      ascending rows, bit-identical to matvec_csrcsym1.
+//      cursor copied from colptr; half a wavefront per row, so that a row's
+//      atomics are in flight together);
+//   4. per row, one wavefront orders the column's list by CSRC position, so
+//      the order, and the FP64 result, never depend on the atomics, and adds
+//      y_i = ad_i x_i + row i in CSRC order + column i in ascending rows,
+//      bit-identical to matvec_csrcsym1.
+// On hex8 28^3 (neq 70,644, nad 2.6 M) a call takes 157 us: counts 27,
+// placement 54 (bound by its atomics; 178 with one lane per row), ordering and
+// product 70.  The last replaces an insertion sort of every list by one lane
+// (1,113 us: a serial chain of dependent global loads and stores) and a gather
+// product with one lane per row (98 us, uncoalesced); the call took 1,403 us.
 #include <mutex>
 
 #include "elastic_internal.h"
@@ -124,39 +131,160 @@ __global__ __launch_bounds__(256) void k_scan_add(int n, int32_t* __restrict__ c
   if (i == n) colptr[n] = tot[nb];
 }
 
-// every stored entry into its column's list (any order inside a list)
+// every stored entry into its column's list (any order inside a list); 32
+// lanes per row
 __global__ __launch_bounds__(256) void k_place(int n, const int32_t* __restrict__ ia,
                                                 const int32_t* __restrict__ ja,
                                                 int32_t* __restrict__ cursor,
                                                 int32_t* __restrict__ colk,
                                                 int32_t* __restrict__ colrow) {
-  for (int r = blockIdx.x * 256 + threadIdx.x; r < n; r += gridDim.x * 256)
-    for (int k = ia[r] - 1; k < ia[r + 1] - 1; ++k) {
+  const int sub = threadIdx.x & 31;
+  for (int64_t r = blockIdx.x * 8ll + (threadIdx.x >> 5); r < n; r += (int64_t)gridDim.x * 8) {
+    const int k2 = ia[r + 1] - 1;
+    for (int k = ia[r] - 1 + sub; k < k2; k += 32) {
       const int c = ja[k] - 1;
       if (c < 0 || c >= n) continue;  // as in the count
       const int p = atomicAdd(&cursor[c], 1);
       colk[p] = k;
-      colrow[p] = r;
+      colrow[p] = (int)r;
+    }
+  }
+}
+
+// The list colk[a..b) ordered in place by one wavefront, with its rows
+// (positions ascend with rows): Batcher's merge exchange, valid for any
+// length.  Only lists the register path below cannot hold come here.
+__device__ void sort_list(int a, int b, int32_t* colk, int32_t* colrow) {
+  const int lane = threadIdx.x & 63, len = b - a;
+  for (int64_t p = 1; p < len; p <<= 1)
+    for (int64_t d = p; d >= 1; d >>= 1) {
+      // pairs (i, i + d), i = (d mod p) + 2 d j + (0..d-1), inside one 2p group
+      const int64_t off = d % p;
+      for (int64_t q = lane;; q += 64) {
+        const int64_t i = off + 2 * d * (q / d) + q % d;
+        if (i + d >= len) break;  // i grows with q
+        if (i / (2 * p) == (i + d) / (2 * p)) {
+          const int32_t k0 = colk[a + i], k1 = colk[a + i + d];
+          if (k0 > k1) {
+            const int32_t r0 = colrow[a + i];
+            colk[a + i] = k1;
+            colk[a + i + d] = k0;
+            colrow[a + i] = colrow[a + i + d];
+            colrow[a + i + d] = r0;
+          }
+        }
+      }
+      // the next step reads what other lanes of this wavefront stored
+      __threadfence_block();
+      __builtin_amdgcn_wave_barrier();
     }
 }
 
-// each column's list sorted by CSRC position (insertion sort: the lists of
-// finite element patterns are short); positions ascend with rows
-__global__ __launch_bounds__(256) void k_sort_cols(int n, const int32_t* __restrict__ colptr,
-                                                    int32_t* __restrict__ colk,
-                                                    int32_t* __restrict__ colrow) {
-  for (int j = blockIdx.x * 256 + threadIdx.x; j < n; j += gridDim.x * 256) {
-    const int a = colptr[j], b = colptr[j + 1];
-    for (int q = a + 1; q < b; ++q) {
-      const int k = colk[q], r = colrow[q];
-      int p = q - 1;
-      while (p >= a && colk[p] > k) {
-        colk[p + 1] = colk[p];
-        colrow[p + 1] = colrow[p];
-        --p;
+// y = A x from the transposed lists in any order.  One wavefront takes kCols
+// rows at a time.  Products are formed by all lanes (row entries and list
+// entries are contiguous, so their loads coalesce) and land in LDS in the
+// order of the sum: row entries first, then the list's entries at their rank,
+// found by comparing every key of the list (a broadcast LDS read serves four
+// keys).  One lane per row then adds its products one after the other, since
+// the order of the reference's sums is kept.  Rows with more than kSlots
+// products, or lists of more than 64 entries, are ordered in place and added
+// in pieces of 64.  Eight rows per wavefront: 36 KiB of LDS per workgroup,
+// four workgroups per CU.
+constexpr int kCols = 8, kSlots = 128;
+__global__ __launch_bounds__(256) void k_sort_gather(int n, const int32_t* __restrict__ ia,
+                                                      const int32_t* __restrict__ ja,
+                                                      const double* __restrict__ ad,
+                                                      const double* __restrict__ al,
+                                                      const int32_t* __restrict__ colptr,
+                                                      int32_t* colk, int32_t* colrow,
+                                                      const double* __restrict__ x,
+                                                      double* __restrict__ y) {
+#pragma clang fp contract(off)
+  __shared__ double prod[4][kCols][kSlots + 1];  // (odd stride: the summing lanes' banks differ)
+  __shared__ __align__(16) int32_t keys[4][kCols][64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  double(*pr)[kSlots + 1] = prod[w];
+  for (int64_t i0 = ((int64_t)blockIdx.x * 4 + w) * kCols; i0 < n;
+       i0 += (int64_t)gridDim.x * 4 * kCols) {
+    const int nc = (int)min((int64_t)kCols, n - i0);
+    // lane c < nc holds the bounds of row i0 + c and of its list
+    int k1 = 0, k2 = 0, c1 = 0, c2 = 0;
+    if (lane < nc) {
+      k1 = ia[i0 + lane] - 1;
+      k2 = ia[i0 + lane + 1] - 1;
+      c1 = colptr[i0 + lane];
+      c2 = colptr[i0 + lane + 1];
+    }
+    const bool fits = (int64_t)(k2 - k1) + (c2 - c1) <= kSlots && k2 - k1 <= 64 && c2 - c1 <= 64;
+    int key[kCols];
+    double pc[kCols];
+#pragma unroll
+    for (int c = 0; c < kCols; ++c) {
+      const bool f = __shfl((int)fits, c, 64) != 0 && c < nc;
+      const int a1 = __shfl(k1, c, 64), a2 = f ? __shfl(k2, c, 64) : a1;
+      const int b1 = __shfl(c1, c, 64), b2 = f ? __shfl(c2, c, 64) : b1;
+      key[c] = INT32_MAX;
+      pc[c] = 0.0;
+      if (b1 + lane < b2) {
+        key[c] = colk[b1 + lane];
+        pc[c] = al[key[c]] * x[colrow[b1 + lane]];
       }
-      colk[p + 1] = k;
-      colrow[p + 1] = r;
+      keys[w][c][lane] = key[c];
+      if (a1 + lane < a2) pr[c][lane] = al[a1 + lane] * x[ja[a1 + lane] - 1];
+    }
+    __builtin_amdgcn_wave_barrier();
+    __threadfence_block();
+#pragma unroll
+    for (int c = 0; c < kCols; ++c) {
+      const int a1 = __shfl(k1, c, 64), a2 = __shfl(k2, c, 64);
+      const int b1 = __shfl(c1, c, 64), b2 = __shfl(c2, c, 64);
+      if (!__shfl((int)fits, c, 64) || c >= nc) continue;
+      int rank = 0;
+      const int4* kv = reinterpret_cast<const int4*>(keys[w][c]);
+      for (int q = 0; 4 * q < b2 - b1; ++q) {  // (entries past the end hold INT32_MAX)
+        const int4 v = kv[q];
+        rank += (v.x < key[c]) + (v.y < key[c]) + (v.z < key[c]) + (v.w < key[c]);
+      }
+      if (b1 + lane < b2) pr[c][a2 - a1 + rank] = pc[c];
+    }
+    __builtin_amdgcn_wave_barrier();
+    __threadfence_block();
+    if (lane < nc && fits) {
+      const int m = (k2 - k1) + (c2 - c1);
+      double t = ad[i0 + lane] * x[i0 + lane];
+      int q = 0;
+      for (; q + 8 <= m; q += 8) {  // eight LDS reads in flight, added in order
+        double v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = pr[lane][q + j];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) t = t + v[j];
+      }
+      for (; q < m; ++q) t = t + pr[lane][q];
+      y[i0 + lane] = t;
+    }
+    __builtin_amdgcn_wave_barrier();
+    for (int c = 0; c < nc; ++c) {  // rows and lists that do not fit
+      if (__shfl((int)fits, c, 64)) continue;
+      const int a1 = __shfl(k1, c, 64), a2 = __shfl(k2, c, 64);
+      const int b1 = __shfl(c1, c, 64), b2 = __shfl(c2, c, 64);
+      sort_list(b1, b2, colk, colrow);
+      double t = ad[i0 + c] * x[i0 + c];
+      for (int part = 0; part < 2; ++part) {
+        const int s1 = part ? b1 : a1, s2 = part ? b2 : a2;
+        for (int s = s1; s < s2; s += 64) {
+          const int m = min(64, s2 - s);
+          if (lane < m)
+            pr[0][lane] = part ? al[colk[s + lane]] * x[colrow[s + lane]]
+                               : al[s + lane] * x[ja[s + lane] - 1];
+          __builtin_amdgcn_wave_barrier();
+          __threadfence_block();
+          for (int q = 0; q < m; ++q) t = t + pr[0][q];
+          __builtin_amdgcn_wave_barrier();
+          __threadfence_block();
+        }
+      }
+      if (lane == 0) y[i0 + c] = t;
     }
   }
 }
@@ -208,12 +336,11 @@ extern "C" int elastic_spmv_csrc_noalloc(int32_t neq, int64_t nad, const int32_t
   hipLaunchKernelGGL(k_scan_add, dim3((neq + 1 + 255) / 256), dim3(256), 0, s, neq, colptr,
                      (const int32_t*)tot, nb, cnt);
   if (nad > 0) {
-    hipLaunchKernelGGL(k_place, dim3(grid_of(neq)), dim3(256), 0, s, neq, ia, ja, cnt, colk,
-                       colrow);
-    hipLaunchKernelGGL(k_sort_cols, dim3(grid_of(neq)), dim3(256), 0, s, neq,
-                       (const int32_t*)colptr, colk, colrow);
+    hipLaunchKernelGGL(k_place, dim3(grid_of(32 * (int64_t)neq)), dim3(256), 0, s, neq, ia, ja,
+                       cnt, colk, colrow);
   }
-  launch_spmv_gather<double>(neq, ia, ja, ad, al, colptr, colk, colrow, x, y, s, nullptr);
+  hipLaunchKernelGGL(k_sort_gather, dim3(grid_of(8 * (int64_t)neq)), dim3(256), 0, s, neq, ia, ja,
+                     ad, al, (const int32_t*)colptr, colk, colrow, x, y);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) {
     fprintf(stderr, "elastic_spmv_csrc_noalloc: %s\n", hipGetErrorString(e));

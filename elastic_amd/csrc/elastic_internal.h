@@ -160,7 +160,8 @@ struct SolveScalars {
   // reliable-update mixed precision (FP32 iteration, FP64 residual replacement)
   double rmax, delta, true_rmr;
   int32_t reliable, upd, skip64, nupd;
-  // BiCGSTAB omega; GMRES: |e(i)| of the last inner step and its norm h(i+1,i)
+  // BiCGSTAB omega; GMRES: |e(i)| of the last inner step and the norm of the
+  // cycle's first vector
   double omega, gm_e, gm_h;
   // progress guard of the mixed methods (device_util.h: progress_guard)
   double last_true;
@@ -170,6 +171,9 @@ struct SolveScalars {
   // batch: restart flags by iteration parity (set when the progress guard
   // hands over to the FP64 operator; the next p update takes beta = 0)
   int32_t restart[2];
+  // GMRES: the cycle's inner steps so far; set once |e(i)| <= econv (the
+  // steps enqueued after that return at once)
+  int32_t gm_ni, gm_done;
 };
 
 constexpr int kRedBlocks = 1024;  // fixed reduction grid (deterministic sums)

@@ -1,6 +1,9 @@
 // 3x3 block-Jacobi set-up on the device, BiCGSTAB and GMRES(k).
 #include <cmath>
 
+#include <algorithm>
+
+#include "spmv_block.h"
 #include "device_util.h"
 #include "elastic_internal.h"
 
@@ -468,12 +471,25 @@ int bicgstab_run(Context* c, bool bdiag, bool fp32_operator, double tol, int max
 
 // ================================================================== GMRES
 // Iters.f:528-808: restarted GMRES(k), left preconditioner M, x0 = 0,
-// econv = tol ||M b||.  Arnoldi with modified Gram-Schmidt (one fused pass per
-// basis vector: w -= h(j,i) g_j together with the partial dot for g_{j+1}),
-// Givens rotations and the back substitution on the device (one block), the
-// x update as one pass over the cycle's basis.  The host reads |e(i)| after
-// every inner step.  Small arrays (column-major like the reference): h
-// (k+1) x k, c(k), s(k), e(k+1), y(k).
+// econv = tol ||M b||.  The Arnoldi basis is orthogonalized by classical
+// Gram-Schmidt done twice: all of a step's products with the basis are formed
+// in one pass, instead of the chain of one pass per basis vector that the
+// modified form needs, and the second pass brings the loss of orthogonality
+// to rounding level (the modified form's grows with the condition of the
+// Krylov vectors).  One inner step is six launches:
+//   product -> w = M A g_i and h1 = G.w -> w -= G h1 and h2 = G.w
+//     -> w -= G h2 and w.w -> g_{i+1} = w / ||w||, Givens rotations
+// (with the block preconditioner the partials are merged in a pass before the
+// second).  The rotations, the stop test and the back substitution run on the
+// device; once |e(i)| <= econv the steps already enqueued return at once, and
+// the host looks every check_every steps.  Bytes of a step: three passes over
+// the basis (the products after an update find its rows in cache), where the
+// modified form's chain moved four vectors per basis vector.  On hex8 17^3
+// (16,524 equations, GMRES(50)) a step bound by the chain's launches and a host
+// read took 155 us; these passes take 36 us (product 6.7, w and h1 7.7, the two
+// updates 9.1 and 6.2, step 4.2): 132 -> 30.6 ms for 849 steps.
+// Small arrays (column-major like the reference): h (k+1) x k, c(k), s(k),
+// e(k+1), y(k).
 
 struct GmSmall {
   double *h, *c, *s, *e, *y;
@@ -520,43 +536,206 @@ __global__ __launch_bounds__(kThreads) void k_gm_merge(int n, MergeArgs mg,
   }
 }
 
-// w = M u ; partial w.g1
-__global__ __launch_bounds__(kThreads) void k_gm_mdot(int n, const double* __restrict__ u,
-                                                       const double* __restrict__ m,
-                                                       const double* __restrict__ bm, double* w,
-                                                       const double* __restrict__ g1,
-                                                       double* part) {
-  __shared__ double sh[8];
-  double acc = 0.0;
-  GRID_LOOP(i, n) {
-    const double wi = apply_m(i, n, u, m, bm);
-    w[i] = wi;
-    acc += wi * g1[i];
-  }
-  const double s = block_sum(acc, sh);
-  if (threadIdx.x == 0) part[blockIdx.x] = s;
+// Sum of v over the wavefront, in lane 63 (DPP lane moves, fixed order).
+__device__ __forceinline__ double wave_sum(double v) {
+  v += dpp_move<0x111, 0xF>(v);
+  v += dpp_move<0x112, 0xF>(v);
+  v += dpp_move<0x114, 0xF>(v);
+  v += dpp_move<0x118, 0xF>(v);
+  v += dpp_move<0x142, 0xA>(v);
+  v += dpp_move<0x143, 0xC>(v);
+  return v;
 }
 
-// one MGS step: beta = w.g_j (from the partials); w -= beta g_j; h(j,i) = beta;
-// partial w.g_{j+1} (gnext) or w.w (gnext == null)
-__global__ __launch_bounds__(kThreads) void k_gm_mgs(int n, const double* __restrict__ part_in,
-                                                      double* w, const double* __restrict__ gj,
-                                                      const double* __restrict__ gnext,
-                                                      double* part_out, double* hji) {
-  __shared__ double sh[8];
-  const double beta = grid_sum(part_in, sh);
-  double acc = 0.0;
-  GRID_LOOP(i, n) {
-    const double wi = w[i] - beta * gj[i];
-    w[i] = wi;
-    acc += wi * (gnext ? gnext[i] : wi);
+// Rows of a basis pass: a workgroup of NT lanes is JW groups of RL = NT / JW
+// lanes.  Workgroup b takes rows [b R, (b + 1) R), in pieces of RL EW rows whose
+// w the lanes of every group keep in registers; group q takes the basis
+// vectors 4 (q + JW p) .. + 3, p = 0, 1, ...  (Small systems: four groups of
+// one wavefront, so that a step's loads are a few deep instead of one per
+// basis vector; large ones: one group.)
+struct GmRows {
+  int n, R;
+};
+
+// acc[wave of the group][j] += this wavefront's share of w.g_j for the
+// group's j < i; four basis vectors at a time, so that 4 EW loads are in
+// flight.
+template <int NT, int JW, int EW>
+__device__ __forceinline__ void gm_dots(int i, int n, int end, int r0, const double (&w)[EW],
+                                        const double* __restrict__ g, double* acc) {
+  constexpr int RL = NT / JW;
+  const int lane = threadIdx.x & 63, gt = threadIdx.x % RL;
+  double* a = acc + (size_t)(gt >> 6) * i;
+  for (int j = 4 * (threadIdx.x / RL); j < i; j += 4 * JW) {
+    double d[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int e = 0; e < EW; ++e) {
+        const int r = r0 + e * RL + gt;
+        if (j + q < i && r < end) d[q] += w[e] * g[(size_t)(j + q) * n + r];
+      }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) d[q] = wave_sum(d[q]);
+    if (lane == 63)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (j + q < i) a[j + q] += d[q];
   }
-  const double s = block_sum(acc, sh);
-  if (threadIdx.x == 0) part_out[blockIdx.x] = s;
-  if (blockIdx.x == 0 && threadIdx.x == 0) *hji = beta;
 }
 
-// e(0) = ||g1||: from the partials; sc->gm_h = e(0)
+// the workgroup's shares: part[j gridDim + b] = sum over a group's NW wavefronts
+template <int NT, int NW>
+__device__ __forceinline__ void gm_store(int i, const double* acc, double* part) {
+  __syncthreads();
+  for (int j = threadIdx.x; j < i; j += NT) {
+    double v = 0.0;
+    for (int k = 0; k < NW; ++k) v += acc[(size_t)k * i + j];
+    part[(size_t)j * gridDim.x + blockIdx.x] = v;
+  }
+}
+
+// h[j] = the workgroups' shares of w.g_j in workgroup order (a wavefront takes
+// four j at a time; every workgroup forms the same sums)
+template <int NT>
+__device__ __forceinline__ void gm_sums(int i, const double* __restrict__ part, double* h) {
+  const int lane = threadIdx.x & 63, nb = gridDim.x;
+  for (int j = 4 * (threadIdx.x >> 6); j < i; j += 4 * (NT / 64)) {
+    double v[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int b = lane; b < nb; b += 64)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) v[q] += j + q < i ? part[(size_t)(j + q) * nb + b] : 0.0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v[q] = wave_sum(v[q]);
+    if (lane == 63)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (j + q < i) h[j + q] = v[q];
+  }
+  __syncthreads();
+}
+
+// w = M (t + merged partials) and the shares of h1 = G.w (bm: t is merged
+// already)
+template <int NT, int JW, int EW>
+__global__ __launch_bounds__(NT) void k_gm_first(GmRows rw, int i, MergeArgs mg,
+                                                 const double* __restrict__ t,
+                                                 const double* __restrict__ m,
+                                                 const double* __restrict__ bm,
+                                                 const double* __restrict__ g, double* w,
+                                                 double* part, const SolveScalars* sc) {
+  extern __shared__ double gsh[];
+  constexpr int RL = NT / JW;
+  __shared__ double ws[JW > 1 ? RL * EW : 1];
+  if (sc->gm_done) return;  // (written by an earlier launch only)
+  double* acc = gsh;        // [RL / 64][i]
+  const int gt = threadIdx.x % RL;
+  for (int q = threadIdx.x; q < RL / 64 * i; q += NT) acc[q] = 0.0;
+  __syncthreads();
+  const int end = min(rw.n, (int)(blockIdx.x + 1) * rw.R);
+  for (int r0 = blockIdx.x * rw.R; r0 < end; r0 += RL * EW) {
+    double wv[EW];
+    auto row = [&](int r) {
+      const double v = bm ? apply_m(r, rw.n, t, m, bm) : m[r] * merge_row(mg, r, t[r]);
+      w[r] = v;
+      return v;
+    };
+    if constexpr (JW > 1) {
+      // every row once (the partials' gather is the chain to shorten), shared
+      // with the other groups through LDS
+      __syncthreads();
+      for (int q = threadIdx.x; q < RL * EW; q += NT) ws[q] = r0 + q < end ? row(r0 + q) : 0.0;
+      __syncthreads();
+#pragma unroll
+      for (int e = 0; e < EW; ++e) wv[e] = ws[e * RL + gt];
+    } else {
+#pragma unroll
+      for (int e = 0; e < EW; ++e) {
+        const int r = r0 + e * RL + gt;
+        wv[e] = r < end ? row(r) : 0.0;
+      }
+    }
+    gm_dots<NT, JW, EW>(i, rw.n, end, r0, wv, g, acc);
+  }
+  gm_store<NT, RL / 64>(i, acc, part);
+}
+
+// h = the sums of part_in; w -= G h; LAST: the shares of w.w into part_out[b],
+// else those of the second pass G.w.  Workgroup 0 stores h (LAST: adds it) in
+// the step's column of H.
+template <int NT, int JW, int EW, bool LAST>
+__global__ __launch_bounds__(NT) void k_gm_project(GmRows rw, int i,
+                                                   const double* __restrict__ part_in,
+                                                   const double* __restrict__ g, double* w,
+                                                   double* part_out, double* hcol,
+                                                   const SolveScalars* sc) {
+  extern __shared__ double gsh[];
+  constexpr int RL = NT / JW;
+  __shared__ double gh[JW > 1 ? JW : 1][JW > 1 ? RL * EW : 1];  // the groups' G h
+  if (sc->gm_done) return;
+  double* h = gsh;                              // [i]
+  double* acc = gsh + i;                        // [RL / 64][LAST ? 1 : i]
+  const int na = LAST ? 1 : i;
+  const int gt = threadIdx.x % RL, group = threadIdx.x / RL;
+  for (int q = threadIdx.x; q < RL / 64 * na; q += NT) acc[q] = 0.0;
+  gm_sums<NT>(i, part_in, h);
+  if (blockIdx.x == 0)
+    for (int j = threadIdx.x; j < i; j += NT) hcol[j] = LAST ? hcol[j] + h[j] : h[j];
+  const int end = min(rw.n, (int)(blockIdx.x + 1) * rw.R);
+  double ww = 0.0;
+  for (int r0 = blockIdx.x * rw.R; r0 < end; r0 += RL * EW) {
+    double wv[EW], s[EW];
+#pragma unroll
+    for (int e = 0; e < EW; ++e) {
+      const int r = r0 + e * RL + gt;
+      wv[e] = r < end ? w[r] : 0.0;
+      s[e] = 0.0;
+    }
+    for (int j = 4 * group; j < i; j += 4 * JW) {
+      double v[4][EW];
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int e = 0; e < EW; ++e) {
+          const int r = r0 + e * RL + gt;
+          v[q][e] = j + q < i && r < end ? g[(size_t)(j + q) * rw.n + r] : 0.0;
+        }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const double hj = h[min(j + q, i - 1)];
+#pragma unroll
+        for (int e = 0; e < EW; ++e) s[e] += hj * v[q][e];
+      }
+    }
+    if constexpr (JW > 1) {  // the groups' sums, added in group order
+      __syncthreads();       // (gh of an earlier piece has been read; w has been loaded)
+#pragma unroll
+      for (int e = 0; e < EW; ++e) gh[group][e * RL + gt] = s[e];
+      __syncthreads();
+#pragma unroll
+      for (int e = 0; e < EW; ++e) {
+        s[e] = 0.0;
+#pragma unroll
+        for (int q = 0; q < JW; ++q) s[e] += gh[q][e * RL + gt];
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < EW; ++e) {
+      const int r = r0 + e * RL + gt;
+      wv[e] -= s[e];
+      if (group == 0 && r < end) w[r] = wv[e];
+      ww += wv[e] * wv[e];
+    }
+    if constexpr (!LAST) gm_dots<NT, JW, EW>(i, rw.n, end, r0, wv, g, acc);
+  }
+  if constexpr (LAST) {
+    ww = wave_sum(ww);
+    if (group == 0 && (gt & 63) == 63) acc[gt >> 6] = ww;
+  }
+  gm_store<NT, RL / 64>(na, acc, part_out);
+}
+
+// e(0) = ||g1||: from the partials; sc->gm_h = e(0); a new cycle begins
 __global__ void k_gm_norm0(const double* __restrict__ part, GmSmall a, SolveScalars* sc) {
   __shared__ double sh[8];
   const double d = grid_sum(part, sh);
@@ -564,35 +743,62 @@ __global__ void k_gm_norm0(const double* __restrict__ part, GmSmall a, SolveScal
     a.e[0] = sqrt(d);
     sc->gm_h = a.e[0];
     sc->gm_e = a.e[0];
+    sc->gm_ni = 0;
+    sc->gm_done = 0;
   }
 }
 
-// inner step i (1-based): h(i+1,i) = ||w||, previous rotations on column i,
-// new rotation, e update (Iters.f:691-704)
-__global__ void k_gm_givens(const double* __restrict__ part, int i, int k, GmSmall a,
-                            SolveScalars* sc) {
-  __shared__ double sh[8];
-  const double d = grid_sum(part, sh);
-  if (threadIdx.x == 0) {
-    double* H = a.h + (size_t)(i - 1) * (k + 1);  // column i: H[j-1] = h(j,i)
-    const double nrm = sqrt(d);
-    H[i] = nrm;
-    for (int j = 1; j <= i - 1; ++j) {
-      const double a1 = a.c[j - 1] * H[j - 1] + a.s[j - 1] * H[j];
-      const double a2 = -a.s[j - 1] * H[j - 1] + a.c[j - 1] * H[j];
-      H[j - 1] = a1;
-      H[j] = a2;
+// End of inner step i (1-based): h(i+1,i) = ||w|| from the workgroups' shares,
+// w = w / ||w|| (left unchanged when it is 0); workgroup 0 applies the previous
+// rotations to column i, forms the new one and updates e (Iters.f:691-704).
+template <int NT>
+__global__ __launch_bounds__(NT) void k_gm_step(GmRows rw, int i, int k,
+                                                const double* __restrict__ part, double* w,
+                                                GmSmall a, double econv, SolveScalars* sc) {
+  extern __shared__ double gsh[];  // workgroup 0: column, c and s of the step
+  __shared__ int done;
+  __shared__ double nrm2;
+  if (threadIdx.x == 0) done = sc->gm_done;
+  __syncthreads();
+  // (workgroup 0 of this launch may set the flag while others read it: w is
+  // not used any more then)
+  if (done) return;
+  double* H = a.h + (size_t)(i - 1) * (k + 1);  // column i: H[j-1] = h(j,i)
+  double *hs = gsh, *cs = gsh + i, *ss = gsh + 2 * i;
+  if (blockIdx.x == 0)
+    for (int j = threadIdx.x; j < i; j += NT) {
+      hs[j] = H[j];
+      cs[j] = j < i - 1 ? a.c[j] : 0.0;
+      ss[j] = j < i - 1 ? a.s[j] : 0.0;
     }
-    const double r = sqrt(H[i - 1] * H[i - 1] + H[i] * H[i]);
-    a.c[i - 1] = H[i - 1] / r;
-    a.s[i - 1] = H[i] / r;
-    H[i - 1] = r;
+  gm_sums<NT>(1, part, &nrm2);
+  const double nrm = sqrt(nrm2);
+  const int end = min(rw.n, (int)(blockIdx.x + 1) * rw.R);
+  if (nrm != 0.0)
+    for (int r = blockIdx.x * rw.R + threadIdx.x; r < end; r += NT) w[r] = w[r] / nrm;
+  if (blockIdx.x != 0) return;
+  if (threadIdx.x == 0) {
+    double hj = hs[0];
+    for (int j = 1; j <= i - 1; ++j) {
+      const double hn = hs[j];
+      hs[j - 1] = cs[j - 1] * hj + ss[j - 1] * hn;
+      hj = -ss[j - 1] * hj + cs[j - 1] * hn;
+    }
+    const double r = sqrt(hj * hj + nrm * nrm);
+    const double ci = hj / r, si = nrm / r;
+    a.c[i - 1] = ci;
+    a.s[i - 1] = si;
+    hs[i - 1] = r;
     H[i] = 0.0;
-    a.e[i] = -a.s[i - 1] * a.e[i - 1];
-    a.e[i - 1] = a.c[i - 1] * a.e[i - 1];
-    sc->gm_e = fabs(a.e[i]);
-    sc->gm_h = nrm;
+    const double e0 = a.e[i - 1], e1 = -si * e0;
+    a.e[i] = e1;
+    a.e[i - 1] = ci * e0;
+    sc->gm_e = fabs(e1);
+    sc->gm_ni = i;
+    if (fabs(e1) <= econv) sc->gm_done = 1;
   }
+  __syncthreads();
+  for (int j = threadIdx.x; j < i; j += NT) H[j] = hs[j];
 }
 
 // g = g / *den (den = 0: left unchanged)
@@ -602,26 +808,62 @@ __global__ __launch_bounds__(kThreads) void k_gm_scale(int n, double* g, const d
   GRID_LOOP(i, n) g[i] = g[i] / d;
 }
 
-// back substitution for y(1..ni) (Iters.f:710-717)
-__global__ void k_gm_backsolve(int ni, int k, GmSmall a) {
-  if (threadIdx.x != 0) return;
-  auto H = [&](int r, int c) { return a.h[(size_t)(c - 1) * (k + 1) + (r - 1)]; };
-  a.y[ni - 1] = a.e[ni - 1] / H(ni, ni);
-  for (int i = ni - 1; i >= 1; --i) {
-    double yi = 0.0;
-    for (int j = i + 1; j <= ni; ++j) yi = yi - H(i, j) * a.y[j - 1];
-    a.y[i - 1] = (yi + a.e[i - 1]) / H(i, i);
+// back substitution for y(1..ni) (Iters.f:710-717), column by column so that
+// the rows above advance together; one workgroup, e is used up
+__global__ __launch_bounds__(kThreads) void k_gm_backsolve(int k, GmSmall a,
+                                                           const SolveScalars* sc) {
+  extern __shared__ double es[];
+  const int ni = sc->gm_ni;
+  for (int j = threadIdx.x; j < ni; j += kThreads) es[j] = a.e[j];
+  __syncthreads();
+  for (int j = ni; j >= 1; --j) {
+    const double* H = a.h + (size_t)(j - 1) * (k + 1);  // column j
+    const double yj = es[j - 1] / H[j - 1];
+    for (int r = threadIdx.x; r < j - 1; r += kThreads) es[r] -= H[r] * yj;
+    if (threadIdx.x == 0) a.y[j - 1] = yj;
+    __syncthreads();
   }
 }
 
 // x += sum_j y(j) g_j (Iters.f:721-725), j in reference order
-__global__ __launch_bounds__(kThreads) void k_gm_xupdate(int n, int ni, const double* __restrict__ g,
-                                                          const double* __restrict__ y, double* x) {
+__global__ __launch_bounds__(kThreads) void k_gm_xupdate(int n, const double* __restrict__ g,
+                                                          const double* __restrict__ y, double* x,
+                                                          const SolveScalars* sc) {
+  const int ni = sc->gm_ni;
   GRID_LOOP(i, n) {
     double xi = x[i];
     for (int j = 0; j < ni; ++j) xi = xi + y[j] * g[(size_t)j * n + i];
     x[i] = xi;
   }
+}
+
+// Workgroups and rows of the basis passes: at most 256 workgroups, since every
+// one sums all of them (256 shares of 50 products are 100 KB from L2 each).
+// From 65,536 rows on 1,024 lanes in one group, so that one workgroup per CU
+// keeps enough loads in flight; below, four groups of 64 lanes with as few
+// rows per lane as 256 workgroups allow.
+constexpr int kGmBlocks = 256, kGmLargeRows = 65536;
+struct GmGrid {
+  GmRows rw;
+  int blocks, lanes, ew;
+};
+static GmGrid gm_grid(int n) {
+  GmGrid G;
+  const bool large = n > kGmLargeRows;
+  const int rl = large ? 1024 : 64;
+  G.lanes = large ? 1024 : 256;
+  G.rw.n = n;
+  G.rw.R = ((n + kGmBlocks - 1) / kGmBlocks + rl - 1) / rl * rl;
+  G.ew = G.rw.R >= 3 * rl ? 4 : G.rw.R > rl ? 2 : 1;
+  G.blocks = (n + G.rw.R - 1) / G.rw.R;
+  return G;
+}
+// raises the dynamic LDS limit of a basis kernel once a launch needs it
+template <typename K>
+static void gm_lds(K* kernel, size_t bytes) {
+  if (bytes > 65536)
+    (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                              160 * 1024);
 }
 
 int gmres_run(Context* c, bool bdiag, bool fp32_operator, double tol, int maxit, int k,
@@ -635,8 +877,10 @@ int gmres_run(Context* c, bool bdiag, bool fp32_operator, double tol, int maxit,
     if (c->gm_small) hipFree(c->gm_small);
     c->gm_basis = c->gm_small = nullptr;
     c->gm_k = 0;
+    // the small arrays, then the workgroups' shares of two passes over the basis
     if (hipMalloc((void**)&c->gm_basis, sizeof(double) * (size_t)(k + 1) * n) != hipSuccess ||
-        hipMalloc((void**)&c->gm_small, sizeof(double) * ((size_t)(k + 1) * k + 4 * k + 2)) !=
+        hipMalloc((void**)&c->gm_small,
+                  sizeof(double) * ((size_t)(k + 1) * k + 4 * k + 2 + 2 * (size_t)kGmBlocks * k)) !=
             hipSuccess) {
       (void)hipGetLastError();
       return set_error(c, ELASTIC_OOM, "GMRES basis of " + std::to_string(k + 1) + " vectors");
@@ -648,6 +892,10 @@ int gmres_run(Context* c, bool bdiag, bool fp32_operator, double tol, int maxit,
                                       sizeof(double) * ((size_t)(k + 1) * k + 4 * k + 2), s));
   const dim3 G(kRedBlocks), TB(kThreads);
   double* P[2] = {c->red64, c->red64 + kRedBlocks};
+  const GmGrid gg = gm_grid(n);
+  double* S[2];  // the workgroups' shares: k rows of gg.blocks each
+  S[0] = c->gm_small + (size_t)(k + 1) * k + 4 * k + 2;
+  S[1] = S[0] + (size_t)kGmBlocks * k;
   double *x = c->v64[VX], *b = c->v64[VB], *t = c->v64[VT], *u = c->v64[VU];
   const double* m = c->A64.m;
   const double* bm = bdiag ? solver_bm(c) : nullptr;
@@ -699,27 +947,50 @@ int gmres_run(Context* c, bool bdiag, bool fp32_operator, double tol, int maxit,
     }
     hipLaunchKernelGGL(k_gm_scale, G, TB, 0, s, n, g(1), (const double*)a.e);
     ++cycles;
-    int ni = 0;
     for (int i = 1; i <= k; ++i) {
-      ++nit;
-      ++ni;
-      launch_spmv(c, op32, g(i), t, c->epart64);
-      hipLaunchKernelGGL(k_gm_merge, G, TB, 0, s, n, merge_of(c, c->epart64, epart_f32(c, op32)),
-                         t, u);
+      launch_spmv(c, op32, g(i), t, c->epart64, &sc->gm_done);
+      const MergeArgs mg = merge_of(c, c->epart64, epart_f32(c, op32));
+      if (bm) hipLaunchKernelGGL(k_gm_merge, G, TB, 0, s, n, mg, t, u);
       double* w = g(i + 1);
-      hipLaunchKernelGGL(k_gm_mdot, G, TB, 0, s, n, u, m, bm, w, g(1), P[0]);
-      for (int j = 1; j <= i; ++j)
-        hipLaunchKernelGGL(k_gm_mgs, G, TB, 0, s, n, P[(j - 1) & 1], w, g(j),
-                           j < i ? (const double*)g(j + 1) : nullptr, P[j & 1],
-                           a.h + (size_t)(i - 1) * (k + 1) + (j - 1));
-      hipLaunchKernelGGL(k_gm_givens, dim3(1), TB, 0, s, P[i & 1], i, k, a, sc);
-      hipLaunchKernelGGL(k_gm_scale, G, TB, 0, s, n, w, (const double*)&sc->gm_h);
-      rc = read_scalars();
-      if (rc) return rc;
-      if (hs->gm_e <= econv) break;
+      double* hcol = a.h + (size_t)(i - 1) * (k + 1);
+      const double* gb = c->gm_basis;
+#define ELASTIC_GM(NT, JW, EW)                                                                  \
+  do {                                                                                          \
+    constexpr int NW = NT / JW / 64;                                                            \
+    const size_t l1 = sizeof(double) * NW * (size_t)i, l2 = l1 + sizeof(double) * i;            \
+    gm_lds(k_gm_first<NT, JW, EW>, l1);                                                         \
+    gm_lds(k_gm_project<NT, JW, EW, false>, l2);                                                \
+    hipLaunchKernelGGL((k_gm_first<NT, JW, EW>), dim3(gg.blocks), dim3(NT), l1, s, gg.rw, i,    \
+                       mg, (const double*)(bm ? u : t), m, bm, gb, w, S[0],                     \
+                       (const SolveScalars*)sc);                                                \
+    hipLaunchKernelGGL((k_gm_project<NT, JW, EW, false>), dim3(gg.blocks), dim3(NT), l2, s,     \
+                       gg.rw, i, (const double*)S[0], gb, w, S[1], hcol,                        \
+                       (const SolveScalars*)sc);                                                \
+    hipLaunchKernelGGL((k_gm_project<NT, JW, EW, true>), dim3(gg.blocks), dim3(NT),             \
+                       sizeof(double) * (i + NW), s, gg.rw, i, (const double*)S[1], gb, w,      \
+                       S[0], hcol, (const SolveScalars*)sc);                                    \
+    hipLaunchKernelGGL(k_gm_step<NT>, dim3(gg.blocks), dim3(NT), 3 * sizeof(double) * i, s,     \
+                       gg.rw, i, k, (const double*)S[0], w, a, econv, sc);                      \
+  } while (0)
+      if (gg.lanes == 256 && gg.ew == 1) ELASTIC_GM(256, 4, 1);
+      else if (gg.lanes == 256 && gg.ew == 2) ELASTIC_GM(256, 4, 2);
+      else if (gg.lanes == 256) ELASTIC_GM(256, 4, 4);
+      else if (gg.ew == 1) ELASTIC_GM(1024, 1, 1);
+      else ELASTIC_GM(1024, 1, 4);
+#undef ELASTIC_GM
+      if (i < k && i % std::max(1, c->check_every) == 0) {
+        rc = read_scalars();
+        if (rc) return rc;
+        if (hs->gm_done) break;
+      }
     }
-    hipLaunchKernelGGL(k_gm_backsolve, dim3(1), dim3(64), 0, s, ni, k, a);
-    hipLaunchKernelGGL(k_gm_xupdate, G, TB, 0, s, n, ni, c->gm_basis, (const double*)a.y, x);
+    hipLaunchKernelGGL(k_gm_backsolve, dim3(1), TB, sizeof(double) * k, s, k, a,
+                       (const SolveScalars*)sc);
+    hipLaunchKernelGGL(k_gm_xupdate, G, TB, 0, s, n, (const double*)c->gm_basis,
+                       (const double*)a.y, x, (const SolveScalars*)sc);
+    rc = read_scalars();
+    if (rc) return rc;
+    nit += hs->gm_ni;
     if (!fp32_operator && hs->gm_e <= econv) conv = true;
   }
   if (fp32_operator && !conv && cycles > 0) {

@@ -73,13 +73,15 @@ static void free_layout(Context* c) {
   c->gather = false;
   c->inc_ptr = c->inc_idx = nullptr;
   // (a layout is never freed inside a solve: x and b are in the CSRC order)
-  void* ptrs[] = {c->A32.ad, c->A32.al, c->epart64, c->tdot, c->p32, c->xd, c->bd, c->bm_dev};
+  void* ptrs[] = {c->A32.ad, c->A32.al, c->epart64, c->tdot, c->p32, c->xd, c->bd, c->bm_dev,
+                  c->res_x};
   for (void* p : ptrs)
     if (p) hipFree(p);
   c->A32 = DevMatrix<float>();
   c->epart64 = nullptr;
   c->tdot = nullptr;
   c->p32 = nullptr;
+  c->res_x = nullptr;
   c->xd = c->bd = c->bm_dev = nullptr;
   c->bdiag_set = false;  // its layout-order copy went with the layout
 }
@@ -115,7 +117,9 @@ using namespace elastic;
 // node blocks per tile the layout is built with (tile_blocks 0: by node size)
 static int effective_tile_blocks(const Context* c, int nb) {
   if (c->tile_blocks > 0) return c->tile_blocks;
-  return nb == 3 && c->neq / 3 >= kLargeTileNodes ? kTileBlocks3 : kTileBlocks2;
+  return nb == 3 && (c->neq / 3 >= kLargeTileNodes || c->nad / 9 > kSmallTileBlocks)
+             ? kTileBlocks3
+             : kTileBlocks2;
 }
 
 static bool getenv_is(const char* name, const char* value) {
@@ -263,6 +267,8 @@ static int build_layout(elastic_ctx* x) {
     nepart = (int64_t)nb * L.next_nodes;
     rc = rc ? rc : dalloc(c, &c->tdot, (size_t)L.ntiles);
     rc = rc ? rc : dalloc(c, &c->p32, 4 * vec32_stride(neq));
+    const size_t nres = resident_words(c);
+    if (nres) rc = rc ? rc : dalloc(c, &c->res_x, nres);
   }
   if (nb == 1) {  // FP32 operator of the scalar tiles (the blocked layout has its planes)
     rc = rc ? rc : dalloc(c, &c->A32.ad, neq);
@@ -363,6 +369,11 @@ int elastic_create(elastic_ctx** out, int32_t device) {
     delete x;
     return ELASTIC_HIP_ERROR;
   }
+  if (hipDeviceGetAttribute(&c->ncu, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess)
+    c->ncu = 0;  // (no resident solves)
+  if (hipDeviceGetAttribute(&c->clock_khz, hipDeviceAttributeWallClockRate, device) != hipSuccess ||
+      c->clock_khz <= 0)
+    c->clock_khz = 100000;
   if (const char* ac = getenv("ELASTIC_ACCUM")) {
     c->accum32 = atoi(ac) == 32;
     c->accum32_set = 1;
@@ -510,10 +521,13 @@ static int time_in_solve(elastic_ctx* x, int precision, int iters, double* ms) {
   c->time_stride = 1;
   c->tprod_ms = 0.0;
   c->tprod_n = 0;
+  const bool resident = c->resident;
+  c->resident = false;  // the candidates are products of a launch each
   elastic_stats st;
   int rc = solve_resident(x, ELASTIC_SOLVER_PCG, ELASTIC_PRECOND_DIAG, precision, 1e-300, iters,
                           50, &st);
   *ms = c->tprod_n ? c->tprod_ms / (double)c->tprod_n : 1e300;
+  c->resident = resident;
   c->time_stride = stride;
   c->tprod_ms = tsum;
   c->tprod_n = tn;
@@ -591,6 +605,8 @@ int elastic_get_option(elastic_ctx* x, const char* name, int64_t* value) {
   else if (n == "tune_tiles") *value = c->tune_tiles ? 1 : 0;
   else if (n == "layout_nb") *value = c->gather ? 0 : c->layout_nb;
   else if (n == "node_order") *value = c->blk.d2r ? 1 : 0;
+  else if (n == "resident") *value = c->resident && c->res_x ? 1 : 0;
+  else if (n == "resident_looks") *value = c->resident_looks;
   else return set_error((Context*)c, ELASTIC_BAD_ARG, "unknown option " + n);
   return ELASTIC_OK;
 }
@@ -623,6 +639,11 @@ int elastic_set_option(elastic_ctx* x, const char* name, int64_t value) {
   } else if (n == "check_every") {
     if (value < 1 || value > 4096) return ELASTIC_BAD_ARG;
     c->check_every = (int)value;
+  } else if (n == "resident") {
+    c->resident = value != 0;
+  } else if (n == "resident_looks") {
+    if (value < 0 || value > (1 << 30)) return ELASTIC_BAD_ARG;
+    c->resident_looks = (int)value;
   } else if (n == "time_products") {
     if (value < 0 || value > 4096) return ELASTIC_BAD_ARG;
     c->time_stride = (int)value;

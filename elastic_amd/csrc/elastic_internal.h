@@ -174,7 +174,17 @@ struct SolveScalars {
   // GMRES: the cycle's inner steps so far; set once |e(i)| <= econv (the
   // steps enqueued after that return at once)
   int32_t gm_ni, gm_done;
+  // resident solves (resident.h): a wait for a peer workgroup ran out
+  int32_t lost;
+  // their products timed on the first workgroup: device clock ticks and count
+  int32_t prod_samples;
+  int64_t prod_ticks;
 };
+
+// words of a resident solve's exchange slots (resident.h): eight copies of four
+// rounds of two sums of 256 workgroups, each copy on other memory channels
+constexpr int kResCopies = 8, kResCopyWords = 4 * 2 * 256 + 32;
+constexpr int kResSlotWords = kResCopies * kResCopyWords;
 
 constexpr int kRedBlocks = 1024;  // fixed reduction grid (deterministic sums)
 
@@ -182,8 +192,12 @@ constexpr int kRedBlocks = 1024;  // fixed reduction grid (deterministic sums)
 // (fewer external partials to write and merge; the FP32 operator's fastest
 // size on hex8 100^3); smaller systems and 2-dof nodes keep 512 (more tiles,
 // so more workgroups in flight; the batch's 2-D product holds 2 blocks per
-// lane).
+// lane).  3-dof systems of more than 512 tiles of 512 blocks take 1,024 too:
+// a resident solve then holds two tiles per CU instead of four smaller ones
+// (hex8 30^3, FP64: 9.7 against 12.4 us per iteration; with launches 26.0
+// against 24.7).
 constexpr int kTileBlocks3 = 1024, kTileBlocks2 = 512;
+constexpr int64_t kSmallTileBlocks = 512 * 512;
 constexpr int kLargeTileNodes = 32768;
 
 struct Context {
@@ -221,6 +235,15 @@ struct Context {
   // workspace
   double *epart64 = nullptr, *red64 = nullptr;
   double* tdot = nullptr;  // per-tile shares of p.(A p) (node-blocked layouts)
+  // words that workgroups of a resident solve exchange (resident.h): the slots,
+  // two rounds of external partials, three rounds of a vector; null where no
+  // resident solve fits
+  double* res_x = nullptr;
+  int res_merge = 0;          // entries of the longest merge list of a tile
+  int ncu = 0;                // CUs of the device
+  int clock_khz = 0;          // device clock of the resident products' timing
+  bool resident = true;       // solves that fit on the chip run there
+  int resident_looks = 1 << 22;  // looks at a peer's word before a wait is given up (~1 us each)
   // FP32 vectors of the mixed PCG with the FP32-sum operator (node-blocked):
   // p at p32, r at p32 + vec32_stride(neq), the Jacobi scale after that,
   // then the FP32 increments of x since the last true-residual replacement
@@ -393,6 +416,16 @@ void launch_sum_parts(const double* part, int nsum, double* out, hipStream_t s);
 struct PcgVecs {
   double *x, *r, *p, *q, *b, *m, *bm, *t, *epart;
 };
+// pcg_resident.hip: the same iteration on a system held on the chip.  The plan
+// is the number of tiles per workgroup, 0 when the system, its operator or its
+// preconditioner does not allow it; a launch runs iterations until the solve
+// converges, asks for a true-residual replacement or reaches maxit.
+int pcg_resident_plan(Context* c, bool fp32_operator, bool bdiag, bool v32);
+// doubles of Context::res_x for the layout just built (0: no resident solve)
+size_t resident_words(Context* c);
+hipError_t pcg_resident_launch(Context* c, const PcgVecs& V, bool fp32_operator, int maxit,
+                               double* dslots, int tpw, float* p32, float* r32, float* m32,
+                               float* dx32);
 int pcg_run(Context* c, const PcgVecs& V, bool fp32_operator, double tol, int maxit,
             bool reliable, double delta, double* dslots);
 }  // namespace elastic

@@ -548,8 +548,8 @@ __global__ __launch_bounds__(kThreads) void k_pcg_restart(int n, const double* _
 }
 
 // ------------------------------------------------------------- host side
-int pcg_run(Context* c, const PcgVecs& V, bool fp32_operator, double tol, int maxit,
-            bool reliable, double delta, double* dslots) {
+static int pcg_iterate(Context* c, const PcgVecs& V, bool fp32_operator, double tol, int maxit,
+                       bool reliable, double delta, double* dslots, bool resident) {
   hipStream_t s = c->stream;
   const int n = c->neq;
   const dim3 G(kRedBlocks), TB(kThreads);
@@ -632,7 +632,52 @@ int pcg_run(Context* c, const PcgVecs& V, bool fp32_operator, double tol, int ma
   double rn_hist[kRateWindow + 1];
   int it_hist[kRateWindow + 1];
   int nhist = 0;
-  while (it < maxit) {
+  // the progress guard's hand-over to the FP64 operator after `at` iterations
+  auto hand_over = [&](int at) {
+    op32 = false;
+    if (v32) {  // the FP64 operator and kernels read the FP64 vectors from here on
+      launch_cast<float, double>(n, p32, V.p, s);
+      launch_cast<float, double>(n, r32, V.r, s);
+      v32 = false;
+      r32 = m32 = nullptr;
+    }
+    // restart: r = b - A64 x, p = M^-1 r, FP64 PCG from here on (the
+    // replacement folds the FP32 increments of x, which end there)
+    hipLaunchKernelGGL(k_rel_force, dim3(1), dim3(64), 0, s, sc);
+    replace(at);
+    dx32 = nullptr;
+    hipLaunchKernelGGL(k_pcg_restart, G, TB, 0, s, n, (const double*)V.r, V.m, V.bm, V.p,
+                       pr_next, sc);
+    replacing = false;
+  };
+  // Systems that fit on the chip iterate there (pcg_resident.hip), one call
+  // per true-residual replacement.  The state a call leaves is the one the
+  // loop below starts an iteration from, so what it does not finish (the FP64
+  // operator after a hand-over) goes on there.
+  const int tpw = resident && tdots ? pcg_resident_plan(c, fp32_operator, !jac, v32) : 0;
+  while (tpw > 0 && it < maxit && !done) {
+    const hipError_t e = pcg_resident_launch(c, V, fp32_operator, maxit, dslots, tpw,
+                                             v32 ? p32 : nullptr, r32, m32, dx32);
+    if (e != hipSuccess) {  // not launched: the launches below take over
+      (void)hipGetLastError();
+      break;
+    }
+    if (reliable) replace(0);  // gated; the flexible recurrences do not read its r.z
+    ELASTIC_HIP_CHECK(c, hipMemcpyAsync(c->scal_host, sc, sizeof(SolveScalars),
+                                        hipMemcpyDeviceToHost, s));
+    ELASTIC_HIP_CHECK(c, hipStreamSynchronize(s));
+    if (c->scal_host->lost)  // a workgroup did not arrive: start over without the resident kernel
+      return pcg_iterate(c, V, fp32_operator, tol, maxit, reliable, delta, dslots, false);
+    it = c->scal_host->iter;
+    done = c->scal_host->done != 0;
+    c->tprod_ms += (double)c->scal_host->prod_ticks / c->clock_khz;
+    c->tprod_n += c->scal_host->prod_samples;
+    if (!done && c->scal_host->op64) {
+      hand_over(it);
+      break;
+    }
+  }
+  while (it < maxit && !done) {
     const int chunk = std::min(every, maxit - it);
     const int it0 = it;
     for (int j = 0; j < chunk; ++j, ++it) {
@@ -709,23 +754,7 @@ int pcg_run(Context* c, const PcgVecs& V, bool fp32_operator, double tol, int ma
       done = true;
       break;
     }
-    if (c->scal_host->op64 && op32) {
-      op32 = false;
-      if (v32) {  // the FP64 operator and kernels read the FP64 vectors from here on
-        launch_cast<float, double>(n, p32, V.p, s);
-        launch_cast<float, double>(n, r32, V.r, s);
-        v32 = false;
-        r32 = m32 = nullptr;
-      }
-      // restart: r = b - A64 x, p = M^-1 r, FP64 PCG from here on (the
-      // replacement folds the FP32 increments of x, which end there)
-      hipLaunchKernelGGL(k_rel_force, dim3(1), dim3(64), 0, s, sc);
-      replace(it);
-      dx32 = nullptr;
-      hipLaunchKernelGGL(k_pcg_restart, G, TB, 0, s, n, (const double*)V.r, V.m, V.bm, V.p,
-                         pr_next, sc);
-      replacing = false;
-    }
+    if (c->scal_host->op64 && op32) hand_over(it);
     if (predict && replacing) {
       const SolveScalars& h = *c->scal_host;
       if (h.upd) replace(it);  // asked for during the chunk: runs before the next one
@@ -761,5 +790,9 @@ int pcg_run(Context* c, const PcgVecs& V, bool fp32_operator, double tol, int ma
   return ELASTIC_OK;
 }
 
+int pcg_run(Context* c, const PcgVecs& V, bool fp32_operator, double tol, int maxit,
+            bool reliable, double delta, double* dslots) {
+  return pcg_iterate(c, V, fp32_operator, tol, maxit, reliable, delta, dslots, true);
+}
 
 }  // namespace elastic

@@ -271,7 +271,14 @@ int elastic_set_tile_blocks(elastic_ctx* ctx, int32_t tile_blocks);
  * 6: node-block Jacobi, the inverses of block_precond with the layout's node
  * size, 2x2 in 2-D and 3x3 in 3-D, applied as op_block_precond does),
  * "time_products" (S > 0: PCG brackets the product of every S-th iteration
- * with HIP events on its stream; 0, the default: off),
+ * with HIP events on its stream -- a resident solve reads the device clock
+ * around it on one workgroup; 0, the default: off),
+ * "resident" (1, the default: PCG on systems that fit on the chip -- up to
+ * 1,024 tiles -- runs its iterations in one cooperative kernel that keeps the
+ * matrix in registers; 0: one launch per phase; both give the same method,
+ * their sums in different orders),
+ * "resident_looks" (how often a workgroup of such a kernel looks for a word of
+ * another before it gives up and the solve starts over with launches),
  * "node_order" (1: the node-blocked tiles of a 3-dof layout are compact
  * breadth-first clusters of the node graph, in whose node order the solves
  * iterate -- b and x are exchanged with the caller in the CSRC order as
@@ -301,7 +308,8 @@ int elastic_autotune(elastic_ctx* ctx, int32_t precision, int32_t reps, int32_t*
 /* Current value of a knob of elastic_set_option, or "lanes64" / "lanes32"
  * (lanes per tile of the FP64 / FP32-value product) or "layout_nb" (node
  * block size of the layout, 1 scalar rows, 0 the gather product);
- * "node_order" reads the order of the layout in use (1 compact). */
+ * "node_order" reads the order of the layout in use (1 compact), "resident"
+ * whether solves that the method allows run on the chip. */
 int elastic_get_option(elastic_ctx* ctx, const char* name, int64_t* value);
 
 /* ------------------------------------------------------ batched serving */

@@ -1,13 +1,15 @@
 // Element stiffness and load assembly on gfx950 (Pform.f:1-254, Assbly.f:66-146,
 // Elmlib02.f elmt02..07, Elmlib.f shape functions and Jacobians).
 //
-// Stiffness (isw = 2), one launch per colour.  hex8 with u = 0 (the
-// assembly of K: b - K u = b) takes k_stiffness_hex8: 16 elements per
-// workgroup, Gauss-point geometry formed once and shared in LDS, one lane per
-// (element, node pair, row) forming only the entries the CSRC stores.  The
-// other cases take k_stiffness: one 64-lane wavefront per element, every
-// lane evaluating the Jacobian of each Gauss point itself, the element matrix
-// s(nst,nst) in LDS and p = s u in the reference's order (Elmlib.f:336-369).
+// Stiffness (isw = 2), one launch per colour.  K of hex8 takes
+// k_stiffness_hex8: 16 elements per workgroup, Gauss-point geometry formed once
+// and shared in LDS, one lane per (element, node pair, row) forming only the
+// entries the CSRC stores.  The other kinds, and b -= K u of hex8, take
+// k_stiffness: one 64-lane wavefront per element, the element matrix s(nst,nst)
+// in LDS and p = s u in the reference's order (Elmlib.f:336-369).  (hex8 with u
+// on 50^3 elements used to take k_stiffness for K as well, every lane indexing
+// private copies of the derivatives, which lived in scratch: 530 us per colour
+// against 79 + 43 us for the two kernels now.)
 // Either way the operations and their order are the reference's (FP
 // contraction off), so every entry is bit-identical to its element matrix,
 // and the entries are added to ad/al/b through the element's slot map with
@@ -288,27 +290,38 @@ __global__ __launch_bounds__(64) void k_stiffness(AsmArgs a, int c0, int lhs, in
   double acc[PER];
   for (int q = 0; q < PER; ++q) acc[q] = 0.0;
   double hx[NEN], hy[NEN], hz[NEN], h[NEN];
-  if (KIND == K_HEX8) {
-    for (int lz = 0; lz < 2; ++lz)
-      for (int ly = 0; ly < 2; ++ly)
-        for (int lx = 0; lx < 2; ++lx) {
-          double det;
-          sfhexa8_d(kPG2[lx], kPG2[ly], kPG2[lz], h, hx, hy, hz);
-          if (!jacob3d_d(hx, hy, hz, xl, NEN, &det)) bad = 1;
-          const double w = 1.0 * 1.0 * 1.0 * det;
-          const double wt1 = w * ca;
+  if constexpr (KIND == K_HEX8) {
+    // one lane per Gauss point forms the derivatives and the weight, kept in
+    // LDS; then one lane per node pair (na, nb) sums its nine entries, six
+    // derivatives read per Gauss point
+    __shared__ double dX[8][3][NEN], wt[8];
+    if (tid < 8) {
+      double det;
+      sfhexa8_d(kPG2[tid & 1], kPG2[(tid >> 1) & 1], kPG2[tid >> 2], h, hx, hy, hz);
+      if (!jacob3d_d(hx, hy, hz, xl, NEN, &det)) bad = 1;
+      const double w = 1.0 * 1.0 * 1.0 * det;
+      wt[tid] = w * ca;
 #pragma unroll
-          for (int q = 0; q < PER; ++q) {
-            const int en = tid + 64 * q;
-            if (en < NENT) {
-              const int i = en % NST, j = en / NST;
-              const int na = i / NDF, r = i % NDF, nb = j / NDF, c = j % NDF;
-              acc[q] = acc[q] + term3(true, r, c, hx[na], hy[na], hz[na], hx[nb], hy[nb], hz[nb],
-                                      cb, cc, wt1);
-            }
-          }
-        }
-  } else if (KIND == K_TET4) {
+      for (int n = 0; n < NEN; ++n) {
+        dX[tid][0][n] = hx[n];
+        dX[tid][1][n] = hy[n];
+        dX[tid][2][n] = hz[n];
+      }
+    }
+    __syncthreads();
+    const int na = tid & 7, nb = tid >> 3;
+    for (int gp = 0; gp < 8; ++gp) {
+      const double xi = dX[gp][0][na], yi = dX[gp][1][na], zi = dX[gp][2][na];
+      const double xj = dX[gp][0][nb], yj = dX[gp][1][nb], zj = dX[gp][2][nb];
+      const double w1 = wt[gp];
+#pragma unroll
+      for (int r = 0; r < 3; ++r)
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+          acc[3 * r + c] =
+              acc[3 * r + c] + term3(true, r, c, xi, yi, zi, xj, yj, zj, cb, cc, w1);
+    }
+  } else if constexpr (KIND == K_TET4) {
     double det;
     if (!jtetra4_d(xl, hx, hy, hz, &det, true)) bad = 1;
     const double wt1 = ca * det * kDIV6;
@@ -321,7 +334,7 @@ __global__ __launch_bounds__(64) void k_stiffness(AsmArgs a, int c0, int lhs, in
         acc[q] = term3(false, r, c, hx[na], hy[na], hz[na], hx[nb], hy[nb], hz[nb], cb, cc, wt1);
       }
     }
-  } else if (KIND == K_QUAD4) {
+  } else if constexpr (KIND == K_QUAD4) {
     for (int ly = 0; ly < 2; ++ly)
       for (int lx = 0; lx < 2; ++lx) {
         double det;
@@ -363,10 +376,18 @@ __global__ __launch_bounds__(64) void k_stiffness(AsmArgs a, int c0, int lhs, in
       }
     }
   }
+  if constexpr (KIND == K_HEX8) {
 #pragma unroll
-  for (int q = 0; q < PER; ++q) {
-    const int en = tid + 64 * q;
-    if (en < NENT) s[en] = acc[q];  // s(i,j) at i + NST*j (column-major)
+    for (int r = 0; r < 3; ++r)
+#pragma unroll
+      for (int c = 0; c < 3; ++c)
+        s[3 * (tid & 7) + r + NST * (3 * (tid >> 3) + c)] = acc[3 * r + c];
+  } else {
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+      const int en = tid + 64 * q;
+      if (en < NENT) s[en] = acc[q];  // s(i,j) at i + NST*j (column-major)
+    }
   }
   __syncthreads();
   if (bad) {
@@ -724,17 +745,18 @@ static AsmArgs make_args(Context* c, MeshDev* m) {
 
 template <int KIND>
 static void launch_stiffness(const AsmArgs& a, const MeshDev* m, int lhs, int rhs, hipStream_t s) {
-  // hex8 stiffness with u = 0 (b - K u = b): the pair kernel
-  const bool pairs = KIND == K_HEX8 && lhs && (!rhs || a.u == nullptr) &&
-                     !getenv_flag("ELASTIC_ASM_WAVE");
+  // hex8 stiffness: the pair kernel; b -= K u of hex8 then takes k_stiffness
+  // for its products alone (u = 0: b - K u = b, nothing to do)
+  const bool pairs = KIND == K_HEX8 && lhs && !getenv_flag("ELASTIC_ASM_WAVE");
+  if (pairs && a.u == nullptr) rhs = 0;
   for (int c = 0; c < m->ncolors; ++c) {
     int c0 = m->color_start[c], cnt = m->color_start[c + 1] - c0;
     if (cnt <= 0) continue;
     if (pairs)
       hipLaunchKernelGGL(k_stiffness_hex8, dim3((cnt + kHexE - 1) / kHexE), dim3(256), 0, s, a,
                          c0, cnt);
-    else
-      hipLaunchKernelGGL(k_stiffness<KIND>, dim3(cnt), dim3(64), 0, s, a, c0, lhs, rhs);
+    if (!pairs || rhs)
+      hipLaunchKernelGGL(k_stiffness<KIND>, dim3(cnt), dim3(64), 0, s, a, c0, pairs ? 0 : lhs, rhs);
   }
 }
 

@@ -421,6 +421,11 @@ struct PcgVecs {
 // preconditioner does not allow it; a launch runs iterations until the solve
 // converges, asks for a true-residual replacement or reaches maxit.
 int pcg_resident_plan(Context* c, bool fp32_operator, bool bdiag, bool v32);
+// bicgstab_resident.hip: the FP64 iteration of bicgstab_run in one call, after
+// its initialisation; plan as above
+int bicgstab_resident_plan(Context* c, bool bdiag);
+hipError_t bicgstab_resident_launch(Context* c, const double* bm, const double* rr, int maxit,
+                                    int tpw);
 // doubles of Context::res_x for the layout just built (0: no resident solve)
 size_t resident_words(Context* c);
 hipError_t pcg_resident_launch(Context* c, const PcgVecs& V, bool fp32_operator, int maxit,

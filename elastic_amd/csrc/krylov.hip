@@ -3,7 +3,7 @@
 
 #include <algorithm>
 
-#include "spmv_block.h"
+#include "resident.h"
 #include "device_util.h"
 #include "elastic_internal.h"
 
@@ -400,8 +400,8 @@ __global__ __launch_bounds__(kThreads) void k_bi_pupdate(int n, const double* __
   if (blockIdx.x == 0 && threadIdx.x == 0) sc->beta = beta;
 }
 
-int bicgstab_run(Context* c, bool bdiag, bool fp32_operator, double tol, int maxit, double delta,
-                 KrylovResult* out) {
+static int bicgstab_iterate(Context* c, bool bdiag, bool fp32_operator, double tol, int maxit,
+                            double delta, KrylovResult* out, bool resident) {
   hipStream_t s = c->stream;
   const int n = c->neq;
   const dim3 G(kRedBlocks), TB(kThreads);
@@ -430,6 +430,22 @@ int bicgstab_run(Context* c, bool bdiag, bool fp32_operator, double tol, int max
   const int every = std::max(1, c->check_every);
   bool done = false;
   bool op32 = fp32_operator;  // the progress guard may hand over to the FP64 operator
+  // FP64 systems that fit on the chip iterate there, in one call
+  const int tpw = resident && !reliable ? bicgstab_resident_plan(c, !jac) : 0;
+  if (tpw > 0) {
+    const hipError_t e = bicgstab_resident_launch(c, bm, rr, maxit, tpw);
+    if (e == hipSuccess) {
+      ELASTIC_HIP_CHECK(c, hipMemcpyAsync(c->scal_host, sc, sizeof(SolveScalars),
+                                          hipMemcpyDeviceToHost, s));
+      ELASTIC_HIP_CHECK(c, hipStreamSynchronize(s));
+      if (c->scal_host->lost)  // a workgroup did not arrive: start over with launches
+        return bicgstab_iterate(c, bdiag, fp32_operator, tol, maxit, delta, out, false);
+      it = maxit;
+      done = c->scal_host->done != 0;
+    } else {
+      (void)hipGetLastError();  // not launched
+    }
+  }
   while (it < maxit && !done) {
     const int chunk = std::min(every, maxit - it);
     for (int j = 0; j < chunk; ++j, ++it) {
@@ -467,6 +483,11 @@ int bicgstab_run(Context* c, bool bdiag, bool fp32_operator, double tol, int max
   out->conv = h.conv;
   out->op64_from = h.op64_from;
   return ELASTIC_OK;
+}
+
+int bicgstab_run(Context* c, bool bdiag, bool fp32_operator, double tol, int maxit, double delta,
+                 KrylovResult* out) {
+  return bicgstab_iterate(c, bdiag, fp32_operator, tol, maxit, delta, out, true);
 }
 
 // ================================================================== GMRES
@@ -534,17 +555,6 @@ __global__ __launch_bounds__(kThreads) void k_gm_merge(int n, MergeArgs mg,
     s = merge_row(mg, i, s);
     u[i] = s;
   }
-}
-
-// Sum of v over the wavefront, in lane 63 (DPP lane moves, fixed order).
-__device__ __forceinline__ double wave_sum(double v) {
-  v += dpp_move<0x111, 0xF>(v);
-  v += dpp_move<0x112, 0xF>(v);
-  v += dpp_move<0x114, 0xF>(v);
-  v += dpp_move<0x118, 0xF>(v);
-  v += dpp_move<0x142, 0xA>(v);
-  v += dpp_move<0x143, 0xC>(v);
-  return v;
 }
 
 // Rows of a basis pass: a workgroup of NT lanes is JW groups of RL = NT / JW

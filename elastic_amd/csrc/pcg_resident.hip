@@ -115,7 +115,7 @@ void k_pcg_resident(ResPcg<TV, T, VT, XT> g) {
     double s1[NS];
     const bool timed = g.stride > 0 && threadIdx.x == 0 && iter % g.stride == 0;
     if (timed) ticks -= (long long)wall_clock64();
-    s1[0] = t.product(ep, qt);
+    s1[0] = t.product(ep, qt, t.xs);
     if (timed) {
       ticks += (long long)wall_clock64();
       ++samples;
@@ -172,23 +172,9 @@ void k_pcg_resident(ResPcg<TV, T, VT, XT> g) {
     }
     int e0 = tid;
     asm volatile("" : "+v"(e0));
-    uint32_t ze[Tile::kExt];  // byte offsets of the external entries
-    u64 zw[Tile::kExt];
-#pragma unroll
-    for (int j = 0; j < Tile::kExt; ++j) {
-      const int e = e0 + 256 * j;
-      ze[j] = e < ne ? 8u * (uint32_t)(NB * t.exn[e / NB] + e % NB) : 0u;
-    }
-    if (!res_exchange<NL, NS>(s2, g.slots, 2 * k3 + 1, g.limit, sh, [&]() {
-          bool ok = true;
-#pragma unroll
-          for (int j = 0; j < Tile::kExt; ++j)
-            if (e0 + 256 * j < ne) zw[j] = peer_get(at_byte(zc, ze[j]));
-#pragma unroll
-          for (int j = 0; j < Tile::kExt; ++j)
-            if (e0 + 256 * j < ne) ok &= zw[j] != kResEmpty;
-          return ok;
-        }))
+    ResExternal E;
+    if (!res_exchange<NL, NS>(s2, g.slots, 2 * k3 + 1, g.limit, sh,
+                              [&]() { return t.ext_look(zc, e0, E); }))
       break;
     const double di = s2[0];
     const double beta = FLEX ? -s2[NS - 1] / pq : di / sh.keep[2];
@@ -204,21 +190,9 @@ void k_pcg_resident(ResPcg<TV, T, VT, XT> g) {
         peer_empty(at(zo) + c);
       }
     }
-#pragma unroll
-    for (int j = 0; j < Tile::kExt; ++j) {
-      const int e = e0 + 256 * j;
-      if (e < ne) xe[e] = (T)fma(beta, (double)xe[e], PeerWord<double>::value(zw[j]));
-    }
-    for (int e = e0 + 256 * Tile::kExt; e < ne; e += 256) {
-      const double* p = zc + (int64_t)NB * t.exn[e / NB] + e % NB;
-      u64 w;
-      for (int n = 0; (w = peer_get(p)) == kResEmpty; ++n)
-        if (n > g.limit) {
-          sh.bad = 1;
-          break;
-        }
-      xe[e] = (T)fma(beta, (double)xe[e], PeerWord<double>::value(w));
-    }
+    if (!t.ext_each(zc, e0, E, g.limit,
+                    [&](int e, double ze) { xe[e] = (T)fma(beta, (double)xe[e], ze); }))
+      sh.bad = 1;
     ++iter;
     ++k3;
     const double rn = sqrt(fabs(di)), conv = sh.keep[0];
@@ -289,19 +263,14 @@ static size_t res_words(const DevBlocks& b) {
   return kResSlotWords + 3 * (size_t)b.nn * b.nb + 2 * (size_t)b.next_nodes * b.nb;
 }
 
-static bool res_one_buffer(const Context* c, size_t t_size, int tpw) {
-  return t_size == 8 && c->blk.nblk_max > 512 && tpw == 4;
-}
-// Tiles per workgroup of a resident solve, or 0 when the system does not fit:
-// one workgroup per CU, all resident at once.  Fewest tiles per workgroup that
-// fit, since the tiles of a CU share its LDS pipe: 205 tiles of 512 blocks
-// (hex8 20^3, FP64) take 7.5 us per iteration one to a CU and 8.0 two to a CU.
-static int res_tpw(const Context* c, size_t t_size) {
+// Fewest tiles per workgroup that fit, since the tiles of a CU share its LDS
+// pipe: 205 tiles of 512 blocks (hex8 20^3, FP64) take 7.5 us per iteration one
+// to a CU and 8.0 two to a CU.
+int resident_tpw(const Context* c, size_t t_size, int most, size_t more) {
   const DevBlocks& b = c->blk;
-  for (int tpw = 1; tpw <= kResTiles; tpw *= 2) {
-    const size_t lds =
-        tpw * res_tile_lds(t_size, b.nb, b.ncols_max, b.nblk_max, c->res_merge,
-                           res_one_buffer(c, t_size, tpw));
+  for (int tpw = 1; tpw <= most; tpw *= 2) {
+    const size_t lds = tpw * (more + res_tile_lds(t_size, b.nb, b.ncols_max, b.nblk_max, c->res_merge,
+                                                  res_one_buffer(t_size, b.nblk_max, tpw)));
     if ((b.ntiles + tpw - 1) / tpw <= std::min(c->ncu, kResGroups) &&
         lds + sizeof(ResShared) + 64 <= 160 * 1024)
       return tpw;
@@ -312,26 +281,34 @@ static int res_tpw(const Context* c, size_t t_size) {
 size_t resident_words(Context* c) {
   if (c->layout_nb < 2 || (c->layout_nb == 2 && c->blk.nblk_max > 512)) return 0;
   c->res_merge = res_merge_max(c->blayout);
-  return res_tpw(c, 4) || res_tpw(c, 8) ? res_words(c->blk) : 0;
+  return resident_tpw(c, 4, kResTiles) || resident_tpw(c, 8, kResTiles) ? res_words(c->blk) : 0;
 }
 
-template <typename TV, typename T, typename VT, typename XT, int NB, int PER, int TPW>
-static hipError_t res_launch(Context* c, ResPcg<TV, T, VT, XT>& g) {
-  const auto k = k_pcg_resident<TV, T, VT, XT, NB, PER, TPW>;
-  const size_t lds = TPW * g.tile_lds;
+void resident_clear(Context* c, size_t t_size) {
+  const DevBlocks& b = c->blk;
+  const int64_t n = (int64_t)b.nn * b.nb, next = b.next_nodes * b.nb;
+  const int64_t n64 = kResSlotWords + 3 * n + (t_size == 8 ? 2 * next : 0);
+  hipLaunchKernelGGL(k_res_empty, dim3((unsigned)std::min<int64_t>((n64 + 255) / 256, 1024)),
+                     dim3(256), 0, c->stream, (u64*)c->res_x, n64,
+                     (uint32_t*)(c->res_x + kResSlotWords + 3 * n),
+                     t_size == 4 ? 2 * next : (int64_t)0, c->scal);
+}
+
+hipError_t resident_start(Context* c, const void* kernel, int tpw, size_t lds, void* args) {
   if (lds > 65536) {
-    const hipError_t e = hipFuncSetAttribute(
-        (const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - sizeof(ResShared) - 64);
+    const hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                             160 * 1024 - sizeof(ResShared) - 64);
     if (e != hipSuccess) return e;
   }
-  void* args[] = {&g};
-  return hipLaunchCooperativeKernel((const void*)k, dim3((g.ntiles + TPW - 1) / TPW),
-                                    dim3(256 * TPW), args, (unsigned)lds, c->stream);
+  void* list[] = {args};
+  return hipLaunchCooperativeKernel(kernel, dim3((c->blk.ntiles + tpw - 1) / tpw), dim3(256 * tpw),
+                                    list, (unsigned)lds, c->stream);
 }
 
 template <typename TV, typename T, typename VT, typename XT, int NB>
 static hipError_t res_dispatch(Context* c, ResPcg<TV, T, VT, XT>& g, int tpw) {
-#define ELASTIC_RES(P, W) return res_launch<TV, T, VT, XT, NB, P, W>(c, g)
+#define ELASTIC_RES(P, W) \
+  return resident_start(c, (const void*)k_pcg_resident<TV, T, VT, XT, NB, P, W>, W, W * g.tile_lds, &g)
   if (c->blk.nblk_max <= 512) {
     if (tpw == 1) ELASTIC_RES(2, 1);
     if (tpw == 2) ELASTIC_RES(2, 2);
@@ -356,11 +333,8 @@ static hipError_t res_run(Context* c, const PcgVecs& V, const TV* vals, const TV
                           (T*)(z + 3 * n), z, x, r, p, m, V.bm, dslots, c->scal, next, n,
                           b.ntiles, maxit, limit, c->res_merge, n < kPredictRows ? 2 : 1, c->time_stride,
                           res_tile_lds(sizeof(T), b.nb, b.ncols_max, b.nblk_max, c->res_merge,
-                                       res_one_buffer(c, sizeof(T), tpw))};
-  const int64_t n64 = kResSlotWords + 3 * n + (sizeof(T) == 8 ? 2 * next : 0);
-  hipLaunchKernelGGL(k_res_empty, dim3((unsigned)std::min<int64_t>((n64 + 255) / 256, 1024)),
-                     dim3(256), 0, c->stream, (u64*)c->res_x, n64, (uint32_t*)(z + 3 * n),
-                     sizeof(T) == 4 ? 2 * next : (int64_t)0, c->scal);
+                                       res_one_buffer(sizeof(T), b.nblk_max, tpw))};
+  resident_clear(c, sizeof(T));
   return b.nb == 3 ? res_dispatch<TV, T, VT, XT, 3>(c, g, tpw)
                    : res_dispatch<TV, T, VT, XT, 2>(c, g, tpw);
 }
@@ -372,7 +346,7 @@ int pcg_resident_plan(Context* c, bool fp32_operator, bool bdiag, bool v32) {
   // FP32 sums: only with the FP32 vectors
   const bool f32 = fp32_operator && c->accum32;
   if (f32 && (!v32 || b.nb != 3)) return 0;
-  return res_tpw(c, f32 ? 4 : 8);
+  return resident_tpw(c, f32 ? 4 : 8, kResTiles);
 }
 
 hipError_t pcg_resident_launch(Context* c, const PcgVecs& V, bool fp32_operator, int maxit,

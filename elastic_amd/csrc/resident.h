@@ -170,12 +170,33 @@ __device__ __forceinline__ bool res_exchange(double (&v)[NS], u64* slots, int se
 #pragma unroll
   for (int k = 0; k < NS; ++k)
     v[k] = (sh.sum[k][0] + sh.sum[k][1]) + (sh.sum[k][2] + sh.sum[k][3]);
-  if (lane < kResCopies && wid < NS)
+  if (lane < kResCopies && wid < 2)  // (the round before may have had two sums)
     peer_empty(reinterpret_cast<double*>(
         slots + (size_t)((seq + kResRounds - 1) % kResRounds) * 2 * kResGroups +
         lane * kResCopyWords + wid * kResGroups + blockIdx.x));
   return sh.bad == 0;
 }
+
+// Waits for words of neighbours only: `pend` until it returns true, then a
+// barrier of the workgroup.
+template <typename Pend>
+__device__ __forceinline__ bool res_wait(int limit, ResShared& sh, Pend pend) {
+  for (int n = 0; !pend(); ++n)
+    if (n > limit) {
+      sh.bad = 1;
+      break;
+    }
+  __syncthreads();
+  return sh.bad == 0;
+}
+
+// A vector of the system as its rows' owners send it to the tiles that have
+// them as external columns: entry e = tid + 256 j of the tile's external
+// columns, the first kExt per lane in flight together.
+constexpr int kResExt = 3;
+struct ResExternal {
+  u64 w[kResExt];
+};
 
 // Shared memory of one tile (bytes): x of its local columns, the blocks' row
 // products and transposed products (`one`: one buffer for both, one after the
@@ -204,7 +225,6 @@ inline size_t res_tile_lds(size_t t_size, int nb, int ncols_max, int nblk_max, i
 template <typename TV, typename T, int NB, int PER, bool TIGHT, bool ONE>
 struct ResTile {
   static constexpr int kMerge = TIGHT ? (PER > 2 ? 2 : 4) : 6;  // partial words of a lane in flight
-  static constexpr int kExt = 3;  // external entries of a lane in flight
   uint32_t wr[PER];
   TV vr[PER][NB * NB];
   int I0, nr, nbk, ncols, ext0;
@@ -295,10 +315,10 @@ struct ResTile {
 
   // q = the row node's own-tile rows of A x, x staged in xs; the partials of
   // external columns go to their words for the owners; returns the lane's share
-  // of x.(A x).  Row products and transposed products go to LDS at their row-
+  // of w.(A x), w staged at ws for the tile's local columns (null: 0).  Row products and transposed products go to LDS at their row-
   // and column-sorted positions and one lane per row or column adds its run.
   // Barriers inside: every lane of the workgroup calls it.
-  __device__ __forceinline__ double product(T* epart, T (&q)[NB]) {
+  __device__ __forceinline__ double product(T* epart, T (&q)[NB], const T* ws) {
     int tid = lane_of_tile();
     // the compiler may not keep what it derives from the lane number and the
     // words (LDS addresses, conditions) in registers from call to call: the
@@ -406,10 +426,44 @@ struct ResTile {
           peer_put(at_byte(epart, (uint32_t)(sizeof(T) * NB) * (uint32_t)(ext0 + c - nr)) + r,
                    s[r]);
       }
+      if (ws)
 #pragma unroll
-      for (int r = 0; r < NB; ++r) dacc += (double)s[r] * (double)xs[c * NB + r];
+        for (int r = 0; r < NB; ++r) dacc += (double)s[r] * (double)ws[c * NB + r];
     }
     return dacc;
+  }
+
+  // External entries of the vector z: ext_look() until it returns true, then
+  // ext_each(f) calls f(entry, value) for the lane's entries (false: an entry
+  // beyond the first kResExt did not arrive).
+  __device__ __forceinline__ uint32_t ext_off(int e) const {
+    return 8u * (uint32_t)(NB * exn[e / NB] + e % NB);
+  }
+  __device__ __forceinline__ bool ext_look(const double* z, int e0, ResExternal& E) const {
+    const int ne = (ncols - nr) * NB;
+    bool ok = true;
+#pragma unroll
+    for (int j = 0; j < kResExt; ++j)
+      if (e0 + 256 * j < ne) E.w[j] = peer_get(at_byte(z, ext_off(e0 + 256 * j)));
+#pragma unroll
+    for (int j = 0; j < kResExt; ++j)
+      if (e0 + 256 * j < ne) ok &= E.w[j] != kResEmpty;
+    return ok;
+  }
+  template <typename F>
+  __device__ __forceinline__ bool ext_each(const double* z, int e0, const ResExternal& E, int limit,
+                                           F f) const {
+    const int ne = (ncols - nr) * NB;
+#pragma unroll
+    for (int j = 0; j < kResExt; ++j)
+      if (e0 + 256 * j < ne) f(e0 + 256 * j, PeerWord<double>::value(E.w[j]));
+    for (int e = e0 + 256 * kResExt; e < ne; e += 256) {
+      u64 w;
+      for (int n = 0; (w = peer_get(at_byte(z, ext_off(e)))) == kResEmpty; ++n)
+        if (n > limit) return false;
+      f(e, PeerWord<double>::value(w));
+    }
+    return true;
   }
 
   // The partials of the tile's row nodes.  look() fetches the lane's words,
@@ -449,5 +503,18 @@ struct ResTile {
       for (int r = 0; r < NB; ++r) q[r] += (double)tr[k + r];
   }
 };
+
+// Tiles per workgroup with which the layout's tiles are all held at once, `more`
+// bytes of LDS per tile beside the product's; 0: they do not fit.
+int resident_tpw(const Context* c, size_t t_size, int most, size_t more = 0);
+// tiles whose row and transposed products share one buffer
+inline bool res_one_buffer(size_t t_size, int nblk_max, int tpw) {
+  return t_size == 8 && nblk_max > 512 && tpw == kResTiles;
+}
+// empties every word of Context::res_x that a solve with sums of t_size bytes
+// exchanges, and the call's flags
+void resident_clear(Context* c, size_t t_size);
+// raises the kernel's LDS limit where needed and launches it cooperatively
+hipError_t resident_start(Context* c, const void* kernel, int tpw, size_t lds, void* args);
 
 }  // namespace elastic

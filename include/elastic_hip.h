@@ -274,7 +274,7 @@ int elastic_set_tile_blocks(elastic_ctx* ctx, int32_t tile_blocks);
  * with HIP events on its stream -- a resident solve reads the device clock
  * around it on one workgroup; 0, the default: off),
  * "resident" (1, the default: PCG on systems that fit on the chip -- up to
- * 1,024 tiles -- runs its iterations in one cooperative kernel that keeps the
+ * 1,024 tiles; FP64 BiCGSTAB up to 512 -- runs its iterations in one cooperative kernel that keeps the
  * matrix in registers; 0: one launch per phase; both give the same method,
  * their sums in different orders),
  * "resident_looks" (how often a workgroup of such a kernel looks for a word of

@@ -21,6 +21,14 @@
 // of block_precond / op_block_precond (2x2 in 2-D, 3x3 in 3-D), in FP64
 // or with the FP32 operator (FP32 values; staging and sums in FP64, or in
 // FP32 when the context asks for it) and FP64 true-residual replacement.
+//
+// Instances that fit on the chip (four tiles per workgroup, one workgroup per
+// CU) iterate there (pcg_resident.h) instead of on the lists, side by side in one
+// cooperative launch per step and, when there are more than the chip holds, one
+// after the other, each system with exchange words of its own.  Per batch, lists
+// against resident: 16 plane sections of up to 160^2 elements 66.4 and 30.5 ms,
+// 8 hex8 12^3 7.7 and 3.5, 6 hex8 33^3 mixed 50.8 and 35.5, 8 hex8 40^3 mixed (each
+// fills the chip) 94.3 and 93.5.
 #include <algorithm>
 #include <chrono>
 #include <cmath>
@@ -29,7 +37,7 @@
 #include <vector>
 
 #include "device_util.h"
-#include "spmv_block.h"
+#include "pcg_resident.h"
 
 namespace elastic {
 
@@ -64,6 +72,12 @@ struct BInst {
   SolveScalars* sc;
   int n, nb, nch, cr, fp32, acc32;  // cr: rows per chunk (nb * (kChunk / nb))
   int live, ntiles;  // live: the slot holds an admitted instance (checked first)
+  // instances held on the chip: the exchange words (Context::res_x), external
+  // partials, longest merge list, LDS per tile, looks before giving up
+  double* res_x;
+  int64_t res_next;
+  size_t res_lds;
+  int res_merge, res_looks;
 };
 
 // ---------------------------------------------------------------- kernels
@@ -701,6 +715,8 @@ __global__ void k_bt_init2(const BInst* __restrict__ insts, int slot, double tol
     sc->skip64 = 1;
     sc->nupd = 0;
     sc->pq_tiles = 0.0;
+    sc->lost = 0;
+    sc->res_round = 0;
     progress_init(sc, sqrt(fabs(d)));
     sc->done = (d == 0.0) ? 1 : 0;
   }
@@ -715,9 +731,116 @@ __global__ __launch_bounds__(kThreads) void k_bt_fold(int n, double* x, float* d
   }
 }
 
+// Variants of the instances held on the chip: value, sum and vector types, node
+// block and node blocks per lane.  Four tiles per workgroup whatever else runs, so
+// that sums do not depend on the mix.  Tiles of more than 512 blocks with FP64 sums
+// stay on the lists: two hex8 40^3 would take 39.6 ms instead of 43.9, but eight,
+// one after the other, 148 instead of 115.
+constexpr int kResVariants = 6;
+struct ResWg {
+  int32_t slot, index, count;  // workgroup `index` of the instance's `count` (0: idle)
+};
+// One launch per variant (two cooperative launches on end leave a gap of 20 us);
+// a workgroup takes one instance after the other, each for `iters` iterations.
+template <typename TV, typename T, typename VT, int NB, int PER>
+__global__ __launch_bounds__(256 * kResTiles) void k_bt_resident(const BInst* __restrict__ insts,
+                                                                 const ResWg* __restrict__ wgs,
+                                                                 int passes, int iters) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  __shared__ ResShared sh;
+  for (int k = 0; k < passes; ++k) {
+    const ResWg w = wgs[k * gridDim.x + blockIdx.x];
+    if (w.count == 0) continue;
+    const BInst& I = insts[w.slot];
+    if (!I.live) continue;
+    SolveScalars* sc = I.sc;
+    // (its workgroups all pass here before one of them writes these, except when it is lost)
+    if (sc->done || sc->op64 || sc->lost) continue;
+    ResPcg<TV, T, VT, VT> g;
+    g.a = I.a;
+    g.mg = I.mg;
+    g.n = I.n;
+    g.next = I.res_next;
+    g.slots = reinterpret_cast<u64*>(I.res_x);
+    g.z = I.res_x + kResSlotWords;
+    g.epart = reinterpret_cast<T*>(g.z + 3 * g.n);
+    if constexpr (sizeof(TV) == 8) {
+      g.vals = I.v64;
+      g.diag = I.d64;
+    } else {
+      g.vals = I.v32;
+      g.diag = I.d32;
+    }
+    if constexpr (sizeof(VT) == 8) {
+      g.x = I.x;
+      g.r = I.r;
+      g.p = I.p;
+      g.m = I.m;
+      g.bm = I.bm;
+    } else {
+      g.x = I.dx32;
+      g.r = I.r32;
+      g.p = I.p32;
+      g.m = I.m32;
+      g.bm = nullptr;
+    }
+    g.dslots = I.dslot;
+    g.sc = sc;
+    g.ntiles = I.ntiles;
+    g.maxit = sc->maxit;
+    g.limit = I.res_looks;
+    g.merge_max = I.res_merge;
+    g.every = 2;  // as on the lists: a step starts at an even iteration
+    g.stride = 0;
+    g.iters = sc->res_round + iters;
+    g.tile_lds = I.res_lds;
+    res_pcg<TV, T, VT, VT, NB, PER, kResTiles, true>(g, w.count, w.index, smem, sh);
+    __syncthreads();
+  }
+}
+static const void* resident_kernel(int v) {
+  switch (v) {
+    case 0: return (const void*)k_bt_resident<double, double, double, 2, 2>;
+    case 1: return (const void*)k_bt_resident<double, double, double, 3, 2>;
+    case 2: return (const void*)k_bt_resident<float, double, double, 2, 2>;
+    case 3: return (const void*)k_bt_resident<float, double, double, 3, 2>;
+    case 4: return (const void*)k_bt_resident<float, float, float, 3, 2>;
+    default: return (const void*)k_bt_resident<float, float, float, 3, 4>;
+  }
+}
+// LDS of one of its tiles
+static size_t resident_lds(const Context* c, bool f32) {
+  return res_tile_lds(f32 ? 4 : 8, c->blk.nb, c->blk.ncols_max, c->blk.nblk_max, c->res_merge, false);
+}
+// the variant of an instance; -1: it iterates on the lists
+static int resident_variant(const Context* c, bool mixed, bool v32, int ncu) {
+  const DevBlocks& b = c->blk;
+  if (!c->resident || !c->res_x || (mixed && c->accum32 && !v32)) return -1;
+  const bool f32 = mixed && c->accum32;
+  if ((b.nb == 2 && f32) || (b.nblk_max > 512 && !f32)) return -1;
+  if ((b.ntiles + kResTiles - 1) / kResTiles > std::min(ncu, kResGroups)) return -1;
+  if (kResTiles * resident_lds(c, f32) + sizeof(ResShared) + 64 > 160 * 1024) return -1;
+  if (f32) return b.nblk_max > 512 ? 5 : 4;
+  return (mixed ? 2 : 0) + (b.nb == 3 ? 1 : 0);
+}
+
+// every word of an instance says that it has not arrived (resident.h); later
+// steps find the words as the step before left them
+__global__ __launch_bounds__(256) void k_bt_res_empty(const BInst* __restrict__ insts, int slot) {
+  const BInst& I = insts[slot];
+  const bool f32 = I.fp32 && I.acc32;
+  const int64_t n64 = kResSlotWords + 3 * (int64_t)I.n + (f32 ? 0 : 2 * I.res_next);
+  const int64_t n32 = f32 ? 2 * I.res_next : 0;
+  u64* w64 = reinterpret_cast<u64*>(I.res_x);
+  uint32_t* w32 = reinterpret_cast<uint32_t*>(I.res_x + kResSlotWords + 3 * (int64_t)I.n);
+  const int64_t i0 = (int64_t)blockIdx.x * 256 + threadIdx.x, st = (int64_t)gridDim.x * 256;
+  for (int64_t k = i0; k < n64; k += st) w64[k] = kResEmpty;
+  for (int64_t k = i0; k < n32; k += st) w32[k] = kResEmpty32;
+}
+
 // done flags / iterations of the active slots for the host
 struct BStatus {
-  int32_t done, status, iter, nupd, op64_from;
+  int32_t done, status, iter, nupd, op64_from, lost;
 };
 __global__ void k_bt_status(const BInst* __restrict__ insts, const int32_t* __restrict__ slots,
                             const int32_t* __restrict__ count, BStatus* out) {
@@ -725,11 +848,11 @@ __global__ void k_bt_status(const BInst* __restrict__ insts, const int32_t* __re
   for (int w = blockIdx.x * blockDim.x + threadIdx.x; w < ns; w += gridDim.x * blockDim.x) {
     const BInst& I = insts[slots[w]];
     if (!I.live) {
-      out[w] = BStatus{0, 0, 0, 0, -1};
+      out[w] = BStatus{0, 0, 0, 0, -1, 0};
       continue;
     }
     const SolveScalars* sc = I.sc;
-    out[w] = BStatus{sc->done, sc->status, sc->iter, sc->nupd, sc->op64_from};
+    out[w] = BStatus{sc->done, sc->status, sc->iter, sc->nupd, sc->op64_from, sc->lost};
   }
 }
 
@@ -751,6 +874,9 @@ struct elastic_batch {
     int64_t tag = 0;
     int ntiles = 0, nch = 0;
     size_t lds = 0;
+    int res = -1;  // its variant on the chip (-1: it iterates on the lists)
+    double tol = 0.0;
+    int maxit = 0;
     std::chrono::steady_clock::time_point t0;
   };
   std::vector<Slot> slots;
@@ -776,7 +902,18 @@ struct elastic_batch {
   int sgrid[kVariants] = {0}, graph_sgrid[kVariants] = {0};
   int ncu = 0;
   int vgrid = 0, graph_vgrid = 0;  // size class of the vector list (one chunk per workgroup)
-  BStatus *d_status = nullptr, *h_status = nullptr;  // h_status pinned
+  // instances held on the chip: the launches of a step and their workgroups,
+  // pass by pass
+  struct ResLaunch {
+    int variant, first, groups, passes;
+    size_t lds;
+  };
+  std::vector<ResLaunch> res_launches;
+  std::vector<ResWg> h_rwgs;
+  ResWg* d_rwgs = nullptr;
+  size_t rwgs_cap = 0;
+  unsigned res_mixed = 0;  // bits 9 / 10 as in mask
+  BStatus* h_status = nullptr;  // pinned: the kernel of the statuses writes it
   bool dirty = true, stepped = false;
   size_t lds = 0, graph_lds = 0;
   hipGraphExec_t gexec = nullptr;
@@ -813,6 +950,21 @@ static void launch_dyn_spmv(elastic_batch* b, int nb3, int mode) {
                        b->d_insts, b->d_dyn, mode);
 }
 
+// true residuals where asked (instances at an even iteration); `mask`: bits 9 / 10
+static void replace_residuals(elastic_batch* b, unsigned mask) {
+  hipStream_t s = b->stream;
+  const dim3 TB(kThreads);
+  const int32_t* scount = b->d_counts + kVariants + 1;
+  hipLaunchKernelGGL(k_bt_dyn_list, dim3(1), dim3(256), 0, s, b->d_insts, b->d_slist, scount,
+                     b->d_dyn, 1);
+  for (int nb3 = 0; nb3 < 2; ++nb3)
+    if (mask & (nb3 ? 0x400u : 0x200u)) {
+      launch_dyn_spmv(b, nb3, 1);
+      hipLaunchKernelGGL(k_bt_dyn_resid, dim3(kDynGrid), TB, 0, s, b->d_insts, b->d_dyn, nb3);
+    }
+  hipLaunchKernelGGL(k_bt_rel_finish, dim3(kMaxSlots), TB, 0, s, b->d_insts, b->d_slist, scount, 0);
+}
+
 // one PCG iteration of every active instance; `it` is the iteration index in
 // the step (its parity selects the r.Mr slot)
 static void enqueue_iteration(elastic_batch* b, int it) {
@@ -842,17 +994,86 @@ static void enqueue_iteration(elastic_batch* b, int it) {
   hipLaunchKernelGGL(k_bt_sum_shares, dim3(kMaxSlots), TB, 0, s, b->d_insts, b->d_slist, scount);
   hipLaunchKernelGGL(k_bt_update, dim3(b->vgrid), TB, 0, s, b->d_insts, b->d_vwork, vcount, cur);
   hipLaunchKernelGGL(k_bt_pupdate, dim3(b->vgrid), TB, 0, s, b->d_insts, b->d_vwork, vcount, cur);
-  if (cur == 1 && mixed) {  // every second iteration: true residuals where asked
-    hipLaunchKernelGGL(k_bt_dyn_list, dim3(1), dim3(256), 0, s, b->d_insts, b->d_slist, scount,
-                       b->d_dyn, 1);
-    for (int nb3 = 0; nb3 < 2; ++nb3)
-      if (b->mask & (nb3 ? 0x400u : 0x200u)) {
-        launch_dyn_spmv(b, nb3, 1);
-        hipLaunchKernelGGL(k_bt_dyn_resid, dim3(kDynGrid), TB, 0, s, b->d_insts, b->d_dyn, nb3);
+  if (cur == 1 && mixed) replace_residuals(b, b->mask);  // every second iteration
+}
+
+static int set_lds_limit(elastic_batch* b);
+
+// Packs the instances held on the chip, one launch per variant and at most one
+// workgroup per CU, the largest first, into as few passes as hold them.
+static int pack_resident(elastic_batch* b) {
+  b->res_launches.clear();
+  b->h_rwgs.clear();
+  b->res_mixed = 0;
+  const int cap = std::min(b->ncu, kResGroups);
+  auto groups = [&](int k) { return (b->slots[k].ntiles + kResTiles - 1) / kResTiles; };
+  for (int v = 0; v < kResVariants; ++v) {
+    std::vector<int> ks;
+    for (int k = 0; k < b->max_slots; ++k)
+      if (b->slots[k].used && b->slots[k].res == v) ks.push_back(k);
+    if (ks.empty()) continue;
+    std::stable_sort(ks.begin(), ks.end(), [&](int p, int q) { return groups(p) > groups(q); });
+    std::vector<std::vector<int>> bins;
+    std::vector<int> room;
+    for (int k : ks) {
+      size_t i = 0;
+      while (i < bins.size() && room[i] < groups(k)) ++i;
+      if (i == bins.size()) {
+        bins.emplace_back();
+        room.push_back(cap);
       }
-    hipLaunchKernelGGL(k_bt_rel_finish, dim3(kMaxSlots), TB, 0, s, b->d_insts, b->d_slist,
-                       scount, 0);
+      bins[i].push_back(k);
+      room[i] -= groups(k);
+      if (b->h_insts[k].fp32) b->res_mixed |= b->h_insts[k].nb == 3 ? 0x400u : 0x200u;
+    }
+    int most = 0;
+    for (int r : room) most = std::max(most, cap - r);
+    elastic_batch::ResLaunch L{v, (int)b->h_rwgs.size(), most, (int)bins.size(), 0};
+    for (const auto& bin : bins) {
+      for (int k : bin) {
+        L.lds = std::max(L.lds, kResTiles * b->h_insts[k].res_lds);
+        for (int i = 0; i < groups(k); ++i) b->h_rwgs.push_back(ResWg{k, i, groups(k)});
+      }
+      while ((b->h_rwgs.size() - L.first) % most) b->h_rwgs.push_back(ResWg{0, 0, 0});
+    }
+    b->res_launches.push_back(L);
   }
+  if (b->h_rwgs.empty()) return ELASTIC_OK;
+  if (b->h_rwgs.size() > b->rwgs_cap) {
+    if (b->d_rwgs) hipFree(b->d_rwgs);
+    b->d_rwgs = nullptr;
+    b->rwgs_cap = 0;
+    const size_t nc = std::max<size_t>(2 * b->h_rwgs.size(), 1024);
+    if (hipMalloc((void**)&b->d_rwgs, nc * sizeof(ResWg)) != hipSuccess)
+      return berr(b, ELASTIC_OOM, "batch workgroup list");
+    b->rwgs_cap = nc;
+  }
+  BATCH_HIP(b, hipMemcpyAsync(b->d_rwgs, b->h_rwgs.data(), b->h_rwgs.size() * sizeof(ResWg),
+                              hipMemcpyHostToDevice, b->stream));
+  return ELASTIC_OK;
+}
+
+// the step of the instances held on the chip, then the true residuals they
+// stopped for
+static int step_resident(elastic_batch* b) {
+  hipStream_t s = b->stream;
+  for (const auto& L : b->res_launches) {
+    const void* f = resident_kernel(L.variant);
+    if (L.lds > 65536)
+      BATCH_HIP(b, hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       160 * 1024 - sizeof(ResShared) - 64));
+    const BInst* insts = b->d_insts;
+    const ResWg* wgs = b->d_rwgs + L.first;
+    int passes = L.passes, iters = b->iters;
+    void* args[] = {&insts, &wgs, &passes, &iters};
+    BATCH_HIP(b, hipLaunchCooperativeKernel(f, dim3(L.groups), dim3(256 * kResTiles), args,
+                                            (unsigned)L.lds, s));
+  }
+  if (!b->res_mixed) return ELASTIC_OK;
+  int rc = set_lds_limit(b);
+  if (rc) return rc;
+  replace_residuals(b, b->res_mixed);
+  return ELASTIC_OK;
 }
 
 static int set_lds_limit(elastic_batch* b) {
@@ -880,6 +1101,8 @@ static int upload_lists(elastic_batch* b) {
     if (!S.used) continue;
     const BInst& I = b->h_insts[k];
     b->h_slist.push_back(k);
+    lds = std::max(lds, S.lds);
+    if (S.res >= 0) continue;
     const int v0 = I.nb == 3 ? 3 : 0;
     // FP64 instances on the FP64 list; mixed ones on an FP32 list (their FP64
     // work goes through the device-built lists)
@@ -890,7 +1113,6 @@ static int upload_lists(elastic_batch* b) {
       mixed_nb |= I.nb == 3 ? 0x400u : 0x200u;
     }
     for (int c = 0; c < S.nch; ++c) b->h_vwork.push_back(((uint32_t)k << 24) | (uint32_t)c);
-    lds = std::max(lds, S.lds);
   }
   unsigned mask = mixed ? 0x100u | mixed_nb : 0u;
   for (int v = 0; v < kVariants; ++v)
@@ -942,6 +1164,8 @@ static int upload_lists(elastic_batch* b) {
                                 hipMemcpyHostToDevice, s));
   BATCH_HIP(b, hipMemcpyAsync(b->d_counts, b->h_counts.data(), b->h_counts.size() * 4,
                               hipMemcpyHostToDevice, s));
+  rc = pack_resident(b);
+  if (rc) return rc;
   // the host vectors must outlive the copies: wait here (admission time only)
   BATCH_HIP(b, hipStreamSynchronize(s));
   if (lds > b->lds) b->lds = lds;
@@ -966,6 +1190,16 @@ static int capture(elastic_batch* b) {
   for (int v = 0; v < kVariants; ++v) b->graph_sgrid[v] = b->sgrid[v];
   b->graph_vgrid = b->vgrid;
   return ELASTIC_OK;
+}
+
+// x = 0 and the method's start
+static void start_instance(elastic_batch* b, int k) {
+  const auto& S = b->slots[k];
+  hipLaunchKernelGGL(k_bt_init, dim3(S.nch), dim3(kThreads), 0, b->stream, b->d_insts, k);
+  hipLaunchKernelGGL(k_bt_init2, dim3(1), dim3(kThreads), 0, b->stream, b->d_insts, k, S.tol,
+                     S.maxit, b->delta);
+  if (S.res >= 0)
+    hipLaunchKernelGGL(k_bt_res_empty, dim3(256), dim3(256), 0, b->stream, b->d_insts, k);
 }
 
 // folds an instance's FP32 increments of x (no-op without them)
@@ -1000,7 +1234,6 @@ int elastic_batch_create(elastic_batch** out, int32_t device, int32_t max_slots,
       hipMalloc((void**)&b->d_insts, sizeof(BInst) * max_slots) != hipSuccess ||
       hipMalloc((void**)&b->d_slist, sizeof(int32_t) * max_slots) != hipSuccess ||
       hipMalloc((void**)&b->d_counts, sizeof(int32_t) * (kVariants + 2)) != hipSuccess ||
-      hipMalloc((void**)&b->d_status, sizeof(BStatus) * max_slots) != hipSuccess ||
       hipMalloc((void**)&b->d_dyn, sizeof(DynList) * kDynLists) != hipSuccess ||
       hipMemset(b->d_dyn, 0, sizeof(DynList) * kDynLists) != hipSuccess ||
       hipHostMalloc((void**)&b->h_status, sizeof(BStatus) * max_slots) != hipSuccess) {
@@ -1033,7 +1266,7 @@ int elastic_batch_destroy(elastic_batch* b) {
   if (b->gexec) hipGraphExecDestroy(b->gexec);
   if (b->graph) hipGraphDestroy(b->graph);
   for (void* p : {(void*)b->d_insts, (void*)b->d_vwork, (void*)b->d_slist, (void*)b->d_counts,
-                  (void*)b->d_status, (void*)b->d_dyn})
+                  (void*)b->d_dyn, (void*)b->d_rwgs})
     if (p) hipFree(p);
   for (uint32_t* p : b->d_sw)
     if (p) hipFree(p);
@@ -1123,18 +1356,27 @@ int elastic_batch_submit(elastic_batch* b, elastic_ctx* x, int32_t precision, do
   I.acc32 = c->accum32 ? 1 : 0;
   I.live = 1;
   I.ntiles = c->blk.ntiles;
+  const int res = resident_variant(c, I.fp32, v32, b->ncu);
+  if (res >= 0) {
+    I.res_x = c->res_x;
+    I.res_next = c->blk.next_nodes * c->layout_nb;
+    I.res_merge = c->res_merge;
+    I.res_looks = c->resident_looks;
+    I.res_lds = resident_lds(c, v32);
+  }
   b->h_insts[k] = I;
   BATCH_HIP(b, hipMemcpyAsync(b->d_insts + k, &b->h_insts[k], sizeof(BInst), hipMemcpyHostToDevice,
                               b->stream));
-  hipLaunchKernelGGL(k_bt_init, dim3(nch), dim3(kThreads), 0, b->stream, b->d_insts, k);
-  hipLaunchKernelGGL(k_bt_init2, dim3(1), dim3(kThreads), 0, b->stream, b->d_insts, k, tol, maxit,
-                     b->delta);
   auto& S = b->slots[k];
+  S.tol = tol;
+  S.maxit = maxit;
+  S.nch = nch;
+  S.res = res;
+  start_instance(b, k);
   S.used = true;
   S.ctx = x;
   S.tag = tag;
   S.ntiles = c->blk.ntiles;
-  S.nch = nch;
   S.lds = tile_lds(c->layout_nb, c->blk.ncols_max, c->blk.nblk_max);
   S.t0 = std::chrono::steady_clock::now();
   b->dirty = true;
@@ -1157,7 +1399,12 @@ int elastic_batch_step(elastic_batch* b) {
     if (rc) return rc;
   }
   if (b->h_slist.empty()) return ELASTIC_OK;
-  if (b->use_graph) {
+  if (!b->res_launches.empty()) {
+    int rc = step_resident(b);
+    if (rc) return rc;
+  }
+  if (b->vgrid == 0) {  // every instance is on the chip
+  } else if (b->use_graph) {
     bool grids = b->vgrid != b->graph_vgrid;
     for (int v = 0; v < kVariants; ++v) grids |= (b->mask & (1u << v)) && b->sgrid[v] != b->graph_sgrid[v];
     if (!b->gexec || b->graph_lds < b->lds || b->graph_mask != b->mask || grids) {
@@ -1171,9 +1418,7 @@ int elastic_batch_step(elastic_batch* b) {
     for (int it = 0; it < b->iters; ++it) enqueue_iteration(b, it);
   }
   hipLaunchKernelGGL(k_bt_status, dim3(1), dim3(256), 0, b->stream, b->d_insts, b->d_slist,
-                     b->d_counts + kVariants + 1, b->d_status);
-  BATCH_HIP(b, hipMemcpyAsync(b->h_status, b->d_status, sizeof(BStatus) * b->h_slist.size(),
-                              hipMemcpyDeviceToHost, b->stream));
+                     b->d_counts + kVariants + 1, b->h_status);
   b->stepped = true;
   return ELASTIC_OK;
 }
@@ -1189,10 +1434,20 @@ int elastic_batch_poll(elastic_batch* b, int64_t* tags, elastic_stats* stats, in
   int nd = 0;
   for (size_t w = 0; w < b->h_slist.size() && nd < cap; ++w) {
     const BStatus& st = b->h_status[w];
-    if (!st.done) continue;
     const int k = b->h_slist[w];
     auto& S = b->slots[k];
     if (!S.used) continue;
+    if (S.res >= 0 && (st.lost || st.op64_from >= 0)) {
+      // a workgroup did not see its peers in time: the instance starts over on
+      // the lists; handed over to the FP64 operator: it goes on there
+      S.res = -1;
+      b->dirty = true;
+      if (st.lost) {
+        start_instance(b, k);
+        continue;
+      }
+    }
+    if (!st.done) continue;
     tags[nd] = S.tag;
     // an instance stopped by maxit still holds FP32 increments of x (a
     // converged one folded them at its last replacement)

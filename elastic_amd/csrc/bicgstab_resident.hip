@@ -44,13 +44,14 @@ __global__ __launch_bounds__(256 * TPW) void k_bicgstab_resident(ResBi g) {
   constexpr int NL = 256 * TPW;
   const int grp = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
   typedef ResTile<double, double, NB, PER, false, false> Tile;
-  const int tid = Tile::lane_of_tile();
+  const int tid = Tile::lane_of_tile(threadIdx.x);
   SolveScalars* sc = g.sc;
   if (sc->done) return;  // (no workgroup writes it before all have passed here)
   if (threadIdx.x == 0) sh.bad = 0;
   Tile t;
   unsigned char* mem = smem + grp * g.tile_lds;
-  t.load(g.a, blockIdx.x * TPW + grp, g.ntiles, g.vals, g.diag, g.mg, g.merge_max, mem);
+  t.load(g.a, blockIdx.x * TPW + grp, g.ntiles, g.vals, g.diag, g.mg, g.merge_max, mem,
+         threadIdx.x);
   double* r0s = reinterpret_cast<double*>(mem + g.prod_lds);  // r0 of the local columns
   const bool own = tid < t.nr;
   uint32_t i0 = (uint32_t)(NB * (t.I0 + (own ? tid : 0)));
@@ -96,7 +97,8 @@ __global__ __launch_bounds__(256 * TPW) void k_bicgstab_resident(ResBi g) {
     int pe = tid;
     s[0] = t.product(ep1, vv, r0s);
     double s1[1] = {s[0]};
-    if (!res_exchange<NL, 1>(s1, g.slots, seq++, g.limit, sh, [&]() { return t.look(ep1, pe); }))
+    if (!res_exchange<NL, 1>(s1, g.slots, threadIdx.x, gridDim.x, blockIdx.x, seq++, g.limit, sh,
+                             [&]() { return t.look(ep1, pe); }))
       break;
     const double vr0 = s1[0];
     // a zero or non-finite denominator, or a non-finite r.r0: every lane sees it
@@ -127,7 +129,7 @@ __global__ __launch_bounds__(256 * TPW) void k_bicgstab_resident(ResBi g) {
     int e0 = tid;
     asm volatile("" : "+v"(e0));
     ResExternal E;
-    if (!res_exchange<NL, 1>(s1, g.slots, seq++, g.limit, sh,
+    if (!res_exchange<NL, 1>(s1, g.slots, threadIdx.x, gridDim.x, blockIdx.x, seq++, g.limit, sh,
                              [&]() { return t.ext_look(z2, e0, E); }))
       break;
     ++iter;
@@ -162,7 +164,9 @@ __global__ __launch_bounds__(256 * TPW) void k_bicgstab_resident(ResBi g) {
         s[1] += tv[c] * tv[c];
       }
     }
-    if (!res_exchange<NL, 2>(s, g.slots, seq++, g.limit, sh, []() { return true; })) break;
+    if (!res_exchange<NL, 2>(s, g.slots, threadIdx.x, gridDim.x, blockIdx.x, seq++, g.limit, sh,
+                             []() { return true; }))
+      break;
     if (s[1] == 0.0 || !isfinite(s[1]) || !isfinite(s[0])) {
       state = 1;
       status = ELASTIC_BREAKDOWN;
@@ -179,7 +183,9 @@ __global__ __launch_bounds__(256 * TPW) void k_bicgstab_resident(ResBi g) {
         s[1] += rv[c] * r0[c];
         peer_empty(at(z2) + c);  // (everyone has formed t from it)
       }
-    if (!res_exchange<NL, 2>(s, g.slots, seq++, g.limit, sh, []() { return true; })) break;
+    if (!res_exchange<NL, 2>(s, g.slots, threadIdx.x, gridDim.x, blockIdx.x, seq++, g.limit, sh,
+                             []() { return true; }))
+      break;
     d = s[0];
     if (!isfinite(d) || !isfinite(s[1])) {
       state = 1;

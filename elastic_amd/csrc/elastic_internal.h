@@ -176,6 +176,7 @@ struct SolveScalars {
   int32_t gm_ni, gm_done;
   // resident solves (resident.h): a wait for a peer workgroup ran out
   int32_t lost;
+  int32_t res_round;  // batch.hip: iterations whose words were exchanged since they were cleared
   // their products timed on the first workgroup: device clock ticks and count
   int32_t prod_samples;
   int64_t prod_ticks;

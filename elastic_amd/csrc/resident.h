@@ -102,7 +102,8 @@ struct ResShared {
   int bad;                       // a wait ran out: every workgroup gives up
 };
 
-// v[k] = its sum over all lanes of all workgroups, the same value everywhere
+// v[k] = its sum over all lanes (this one tid) of the system's workgroups (this
+// one bid of G), the same value everywhere
 // (wavefronts, then workgroups, in a fixed order).  `pend` is called until it
 // returns true, its loads in flight together with those of the sums; it
 // fetches the words this lane waits for in the same exchange.  Round `seq`
@@ -117,10 +118,11 @@ struct ResShared {
 // sixteen gave no more).  Returns false when something did not arrive within `limit`
 // looks.
 template <int NL, int NS, typename Pend>
-__device__ __forceinline__ bool res_exchange(double (&v)[NS], u64* slots, int seq, int limit,
-                                             ResShared& sh, Pend pend) {
+__device__ __forceinline__ bool res_exchange(double (&v)[NS], u64* slots, int tid, int G,
+                                             int bid, int seq, int limit, ResShared& sh,
+                                             Pend pend) {
   constexpr int NW = NL / 64;
-  const int tid = threadIdx.x, lane = tid & 63, G = gridDim.x;
+  const int lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
 #pragma unroll
   for (int k = 0; k < NS; ++k) {
@@ -133,10 +135,10 @@ __device__ __forceinline__ bool res_exchange(double (&v)[NS], u64* slots, int se
     double s = 0.0;
 #pragma unroll
     for (int k = 0; k < NW; ++k) s += sh.red[wid][k];
-    peer_put(reinterpret_cast<double*>(cur + lane * kResCopyWords + wid * kResGroups + blockIdx.x),
+    peer_put(reinterpret_cast<double*>(cur + lane * kResCopyWords + wid * kResGroups + bid),
              s);
   }
-  cur += (blockIdx.x % kResCopies) * kResCopyWords;
+  cur += (bid % kResCopies) * kResCopyWords;
   u64 w[NS];
 #pragma unroll
   for (int k = 0; k < NS; ++k) w[k] = 0;  // (+0.0: lanes without a workgroup)
@@ -173,7 +175,7 @@ __device__ __forceinline__ bool res_exchange(double (&v)[NS], u64* slots, int se
   if (lane < kResCopies && wid < 2)  // (the round before may have had two sums)
     peer_empty(reinterpret_cast<double*>(
         slots + (size_t)((seq + kResRounds - 1) % kResRounds) * 2 * kResGroups +
-        lane * kResCopyWords + wid * kResGroups + blockIdx.x));
+        lane * kResCopyWords + wid * kResGroups + bid));
   return sh.bad == 0;
 }
 
@@ -230,6 +232,7 @@ struct ResTile {
   int I0, nr, nbk, ncols, ext0;
   int nm;      // words of the tile's partials
   int m0, m1;  // those of the row node among them
+  int lane;    // lane of the workgroup
   T *xs, *rw, *tr, *dg;
   int32_t *exn, *mls;
   uint16_t *rps, *sps;
@@ -237,14 +240,15 @@ struct ResTile {
   // Lane of the tile: the wavefronts of a workgroup's tiles are rotated
   // against each other, so that the wavefronts that own rows (the first two
   // of every tile) are spread over the CU's SIMDs.
-  static __device__ __forceinline__ int lane_of_tile() {
-    return (int)((threadIdx.x + 64 * (threadIdx.x >> 8)) & 255);
+  static __device__ __forceinline__ int lane_of_tile(int lane) {
+    return (lane + 64 * (lane >> 8)) & 255;
   }
 
   __device__ __forceinline__ void load(const BlkArgs& a, int t, int ntiles, const TV* vals,
                                        const TV* diag, const MergeArgs& mg, int merge_max,
-                                       unsigned char* smem) {
-    const int tid = lane_of_tile();
+                                       unsigned char* smem, int lane_) {
+    lane = lane_;
+    const int tid = lane_of_tile(lane);
     xs = reinterpret_cast<T*>(smem);
     tr = xs + a.ncols_max * NB;
     const int first = max(a.nblk_max, merge_max) * NB;
@@ -319,7 +323,7 @@ struct ResTile {
   // and column-sorted positions and one lane per row or column adds its run.
   // Barriers inside: every lane of the workgroup calls it.
   __device__ __forceinline__ double product(T* epart, T (&q)[NB], const T* ws) {
-    int tid = lane_of_tile();
+    int tid = lane_of_tile(lane);
     // the compiler may not keep what it derives from the lane number and the
     // words (LDS addresses, conditions) in registers from call to call: the
     // values need them

@@ -1,0 +1,111 @@
+"""Batch instances held on the chip (one cooperative launch per step) against
+the batch's work lists: the same method with sums in another order, so both
+stop at ||r||_M < 1e-11 ||b||_M and x differs by at most the condition number of
+the scaled system (below 1e4 here) times 2e-11; 1e-8 is the library's bar.  An
+instance gives the same bits alone, in a mix and when the chip holds the
+batch's instances only one after the other."""
+import numpy as np
+import pytest
+
+from elastic_amd import mesh as M
+from elastic_amd.solver import FP64, MIXED
+
+pytestmark = pytest.mark.gpu
+
+
+def _systems(kind, sizes, opts):
+    from elastic_amd.system import System
+
+    make = {"hex8": lambda n: M.hex8_cube(n, jitter=0.15, seed=n + 1),
+            "quad4": M.quad4_square, "tria3": M.tria3_square}[kind]
+    out = []
+    for n in sizes:
+        s = System(make(n))
+        for k, v in opts.items():
+            s.ctx.set_option(k, v)
+        s.ctx.upload_rhs(s.b)
+        out.append(s)
+    return out
+
+
+def _run(systems, precision, stagger=0, maxit=20000, iters=8):
+    """{index: (x, stats)}; one instance more every `stagger` steps"""
+    from elastic_amd.serving import Batch
+
+    out, queue, steps = {}, list(range(len(systems))), 0
+    with Batch(0, max_slots=len(systems), iters_per_step=iters) as b:
+        while len(out) < len(systems):
+            while queue and steps >= stagger * queue[0]:
+                k = queue.pop(0)
+                assert b.submit(systems[k].ctx, precision, 1e-11, maxit, k)
+            b.step()
+            steps += 1
+            for k, st in b.poll():
+                out[k] = (systems[k].ctx.download_x(), st)
+            assert steps < 20000
+    return out
+
+
+# (element, sizes, options, precision): tiles alone, of one and of several
+# workgroups, more workgroups than CUs, every operator and vector type
+CASES = [
+    ("quad4", (1, 9, 40), {}, FP64), ("quad4", (33, 12), {"batch_precond": 6}, FP64),
+    ("tria3", (70, 60, 50, 40), {"tile_blocks": 64, "batch_precond": 6}, FP64),
+    ("tria3", (25, 10), {"accum32": 0, "batch_precond": 6}, MIXED),
+    ("hex8", (1, 6, 9), {}, FP64), ("hex8", (7, 5), {"batch_precond": 6}, FP64),
+    ("hex8", (12, 12, 12, 11), {"tile_blocks": 40}, FP64),
+    ("hex8", (8, 5), {"accum32": 0}, MIXED),
+    ("hex8", (8, 11), {"accum32": 1}, MIXED),
+    ("hex8", (12, 11, 12), {"accum32": 1, "tile_blocks": 40}, MIXED),
+    ("hex8", (14, 6), {"accum32": 1, "tile_blocks": 1024}, MIXED),
+    ("hex8", (9,), {"accum32": 1, "batch_precond": 6}, MIXED),  # on the lists
+    ("hex8", (13,), {"tile_blocks": 1024}, FP64),               # on the lists
+]
+
+
+@pytest.mark.parametrize("kind,sizes,opts,precision", CASES)
+def test_matches_the_lists(kind, sizes, opts, precision):
+    systems = _systems(kind, sizes, opts)
+    runs = {}
+    for resident in (0, 1):
+        for s in systems:
+            s.ctx.set_option("resident", resident)
+        print("batch resident", kind, sizes, opts, precision, resident, flush=True)
+        runs[resident] = _run(systems, precision)
+    staggered = _run(systems, precision, stagger=2)
+    for k, s in enumerate(systems):
+        (x0, s0), (x1, s1) = runs[0][k], runs[1][k]
+        assert s0["status"] == s1["status"] == 0
+        assert np.linalg.norm(x1 - x0) <= 1e-8 * np.linalg.norm(x0)
+        slack = 2 if precision == FP64 else max(6, s0["iters"] // 10)
+        assert abs(s1["iters"] - s0["iters"]) <= slack, (s0["iters"], s1["iters"])
+        xa, sa = _run([s], precision)[0]
+        for xb, sb in ((x1, s1), staggered[k]):
+            assert np.array_equal(xa, xb) and sa["iters"] == sb["iters"]
+        s.ctx.close()
+
+
+@pytest.mark.parametrize("precision", [FP64, MIXED])
+def test_limit_of_iterations_and_lost_peers(precision):
+    """maxit ends an instance at the same iteration, odd and even; with no look
+    left for its peers' words an instance starts over on the lists and gives
+    their bits, beside one that stays on the chip."""
+    systems = _systems("hex8", (9, 8), {})
+    for maxit in (7, 24):
+        got = []
+        for resident in (0, 1):
+            systems[0].ctx.set_option("resident", resident)
+            got.append(_run(systems[:1], precision, maxit=maxit)[0])
+        (x0, s0), (x1, s1) = got
+        assert s0["iters"] == s1["iters"] == maxit and s0["status"] == s1["status"] == 2
+        assert np.linalg.norm(x1 - x0) <= 1e-5 * np.linalg.norm(x0)
+    systems[0].ctx.set_option("resident", 0)
+    lists = _run(systems, precision)
+    systems[0].ctx.set_option("resident", 1)
+    systems[0].ctx.set_option("resident_looks", 0)
+    lost = _run(systems, precision)
+    for k in range(2):
+        assert np.array_equal(lists[k][0], lost[k][0])
+        assert lists[k][1]["iters"] == lost[k][1]["iters"]
+    for s in systems:
+        s.ctx.close()

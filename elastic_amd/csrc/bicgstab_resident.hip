@@ -10,7 +10,7 @@
 //   x += omega z, r -= omega t
 //   r.r, r.r0                                               exchange 4, test
 //   p = r + beta (p - omega v), z = M p to its readers (neighbours only)
-// The launch iteration's eleven dependent kernels take 49 us on hex8 24^3, this 19.
+// The launch iteration's eleven dependent kernels take 49 us on hex8 24^3, this 17.8.
 // Words are emptied as in pcg_resident.hip: a z once everyone has published a
 // sum that needed it, and both products' partials have words of their own.
 #include <algorithm>
@@ -124,14 +124,15 @@ __global__ __launch_bounds__(256 * TPW) void k_bicgstab_resident(ResBi g) {
 #pragma unroll
       for (int c = 0; c < NB; ++c) {
         peer_put(at(z2) + c, zv[c]);
-        if (iter > 0) peer_empty(at(z1) + c);  // (everyone has formed v from it)
       }
+    if (iter > 0) t.empty_rows(z1);  // (everyone has formed v from it)
     int e0 = tid;
     asm volatile("" : "+v"(e0));
     ResExternal E;
     if (!res_exchange<NL, 1>(s1, g.slots, threadIdx.x, gridDim.x, blockIdx.x, seq++, g.limit, sh,
                              [&]() { return t.ext_look(z2, e0, E); }))
       break;
+    t.empty_partials(ep1);
     ++iter;
     double d = s1[0];
     if (!isfinite(d)) {
@@ -181,8 +182,9 @@ __global__ __launch_bounds__(256 * TPW) void k_bicgstab_resident(ResBi g) {
         rv[c] = rv[c] - w * tv[c];
         s[0] += rv[c] * rv[c];
         s[1] += rv[c] * r0[c];
-        peer_empty(at(z2) + c);  // (everyone has formed t from it)
       }
+    t.empty_rows(z2);  // (everyone has formed t from it)
+    t.empty_partials(ep2);
     if (!res_exchange<NL, 2>(s, g.slots, threadIdx.x, gridDim.x, blockIdx.x, seq++, g.limit, sh,
                              []() { return true; }))
       break;

@@ -193,15 +193,15 @@ __device__ __forceinline__ void res_pcg(const ResPcg<TV, T, VT, XT>& g, int G, i
     const double di = s2[0];
     const double beta = FLEX ? -s2[NS - 1] / pq : di / sh.keep[2];
     apr = 0.0;
+    // every reader has z of the iteration before, and the partials of this one
+    t.empty_rows(g.z + ((k3 + 2) % 3) * g.n);
+    t.empty_partials(ep);
     if (own) {
-      // (every reader has z of the iteration before)
-      double* zo = g.z + ((k3 + 2) % 3) * g.n;
 #pragma unroll
       for (int c = 0; c < NB; ++c) {
         const T pv = (T)fma(beta, (double)t.xs[tid * NB + c], zv[c]);
         t.xs[tid * NB + c] = pv;
         apr += (double)pv * (double)rv[c];
-        peer_empty(at(zo) + c);
       }
     }
     if (!t.ext_each(zc, e0, E, g.limit,

@@ -4,8 +4,10 @@
 // device.  A launch-per-phase iteration on such systems is bound by its four
 // dependent launches (about 5 us each, whatever they move); here an iteration
 // is bound by two exchanges between the workgroups.  Per iteration, launches
-// against resident: hex8 20^3 FP64 20.9 and 7.5 us, hex8 38^3 mixed 31 and 12.5,
-// quad4 141^2 FP64 18.2 and 6.0, tet4 41^3 x 6 mixed 26.5 and 10.6.
+// against resident: hex8 20^3 FP64 20.9 and 6.8 us, hex8 38^3 mixed 31 and 12.5,
+// quad4 141^2 FP64 18.2 and 5.9, tet4 41^3 x 6 mixed 26.5 and 10.4.  Of the 6.8, the
+// exchanges take 2.1 and 2.3, the product 1.8; with four tiles of 1,024 blocks per CU
+// and FP64 sums (hex8 43^3, 19.6 us) they take 4.2, 5 and 7.5.
 //
 // Everything that crosses workgroups goes through relaxed agent-scope atomics
 // (write-through stores, loads that do not take a line another XCD may hold
@@ -14,8 +16,10 @@
 // workgroups.  A word says itself whether it has arrived: until then it holds
 // a NaN that no computation produces.  So partial sums, external partials and
 // vector entries are all polled at once, one round trip per exchange, and no
-// store is waited for before a flag.  Words are emptied by the side that is
-// known to be the last to need them, and reused only after a later exchange.
+// store is waited for before a flag.  Words are emptied by
+// the side that wrote them, in whole lines (2 to 7% of an iteration against the
+// readers doing it a node at a time), once every reader is known to have them,
+// and reused only after a later exchange.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -200,14 +204,15 @@ struct ResExternal {
   u64 w[kResExt];
 };
 
-// Shared memory of one tile (bytes): x of its local columns, the blocks' row
-// products and transposed products (`one`: one buffer for both, one after the
-// other), the diagonal blocks of the rows, the external nodes, the merge list
+// Shared memory of one tile (bytes): x of its local columns, the blocks'
+// transposed products, the pieces of row products (`one`: one buffer for both,
+// one after the other), the diagonal blocks of the rows, the external nodes, the merge list
 // (merge_max entries) and the row and segment pointers.
+constexpr size_t kResPieces = 256 + kBlkRowsMax;
 inline size_t res_tile_lds(size_t t_size, int nb, int ncols_max, int nblk_max, int merge_max,
                            bool one) {
   // (the partials of a merge list pass through the first buffer)
-  const size_t buf = std::max(nblk_max, merge_max) + (one ? 0 : (size_t)nblk_max);
+  const size_t buf = std::max(nblk_max, merge_max) + (one ? 0 : kResPieces);
   const size_t vals = t_size * (nb * ((size_t)ncols_max + buf) +
                                 (kBlkRowsMax + 1) * (nb * (nb + 1) / 2));
   const size_t ptrs = sizeof(int32_t) * ((size_t)ncols_max + (size_t)merge_max) +
@@ -217,7 +222,9 @@ inline size_t res_tile_lds(size_t t_size, int nb, int ncols_max, int nblk_max, i
 
 // One tile held by 256 lanes: lane tid owns blocks PER tid + i (in row order, so
 // that a lane adds the row products of its consecutive blocks of one row before
-// they go to LDS, about one store per row instead of one per block; the values
+// they go to LDS, about one store per row instead of one per block; lane l's
+// piece of row r goes to place l + r, which makes the pieces of a row one run);
+// the values
 // are read once per call, so their order in memory does not matter) and, below
 // the row count, row node tid.  The partials of the tile's row nodes are one
 // run of the merge list: all lanes fetch them, one word at a time, into LDS,
@@ -253,7 +260,7 @@ struct ResTile {
     tr = xs + a.ncols_max * NB;
     const int first = max(a.nblk_max, merge_max) * NB;
     rw = ONE ? tr : tr + first;
-    dg = ONE ? tr + first : rw + a.nblk_max * NB;
+    dg = ONE ? tr + first : rw + kResPieces * NB;
     exn = reinterpret_cast<int32_t*>(dg + (kBlkRowsMax + 1) * (NB * (NB + 1) / 2));
     mls = exn + a.ncols_max;
     rps = reinterpret_cast<uint16_t*>(mls + merge_max);
@@ -297,30 +304,51 @@ struct ResTile {
     }
   }
 
-  // s += the NB-vectors buf[NB q ..], q0 <= q < q1, in order
+  // s += the NB-vectors buf[NB q ..], q0 <= q < q1, in order.  With ONE buffer a
+  // short last batch is loaded whole (hex8 43^3 20.5 -> 19.6 us per iteration);
+  // elsewhere the wider batches cost more registers than they give.
   static __device__ __forceinline__ void add_run(const T* buf, int q0, int q1, T (&s)[NB]) {
-    constexpr int kU = TIGHT ? 2 : 4;
-    int q = q0;
-    for (; q + kU <= q1; q += kU) {
-      T v[kU][NB];
+    if constexpr (ONE) {
+      constexpr int kU = 2;
+      for (int q = q0; q < q1; q += kU) {
+        T v[kU][NB];
 #pragma unroll
-      for (int j = 0; j < kU; ++j)
+        for (int j = 0; j < kU; ++j) {
+          const int k = min(q + j, q1 - 1);
 #pragma unroll
-        for (int r = 0; r < NB; ++r) v[j][r] = buf[(q + j) * NB + r];
+          for (int r = 0; r < NB; ++r) v[j][r] = buf[k * NB + r];
+        }
 #pragma unroll
-      for (int j = 0; j < kU; ++j)
+        for (int j = 0; j < kU; ++j)
+          if (q + j < q1)
 #pragma unroll
-        for (int r = 0; r < NB; ++r) s[r] += v[j][r];
+            for (int r = 0; r < NB; ++r) s[r] += v[j][r];
+      }
+    } else {
+      constexpr int kU = TIGHT ? 2 : 4;
+      int q = q0;
+      for (; q + kU <= q1; q += kU) {
+        T v[kU][NB];
+#pragma unroll
+        for (int j = 0; j < kU; ++j)
+#pragma unroll
+          for (int r = 0; r < NB; ++r) v[j][r] = buf[(q + j) * NB + r];
+#pragma unroll
+        for (int j = 0; j < kU; ++j)
+#pragma unroll
+          for (int r = 0; r < NB; ++r) s[r] += v[j][r];
+      }
+      for (; q < q1; ++q)
+#pragma unroll
+        for (int r = 0; r < NB; ++r) s[r] += buf[q * NB + r];
     }
-    for (; q < q1; ++q)
-#pragma unroll
-      for (int r = 0; r < NB; ++r) s[r] += buf[q * NB + r];
   }
 
   // q = the row node's own-tile rows of A x, x staged in xs; the partials of
   // external columns go to their words for the owners; returns the lane's share
-  // of w.(A x), w staged at ws for the tile's local columns (null: 0).  Row products and transposed products go to LDS at their row-
-  // and column-sorted positions and one lane per row or column adds its run.
+  // of w.(A x), w staged at ws for the tile's local columns (null: 0).  Pieces of
+  // rows and transposed products go to LDS, row by row and column by column, and
+  // one lane per row or column adds its run.
   // Barriers inside: every lane of the workgroup calls it.
   __device__ __forceinline__ double product(T* epart, T (&q)[NB], const T* ws) {
     int tid = lane_of_tile(lane);
@@ -329,8 +357,8 @@ struct ResTile {
     // values need them
     asm volatile("" : "+v"(tid));
     auto blocks = [&](bool rows, bool cols) {
-      T y[NB];        // row products of the lane's current row, stored at its first block
-      int at = 0, cur = -1;
+      T y[NB];        // row products of the lane's current row
+      int cur = -1;
 #pragma unroll
       for (int i = 0; i < PER; ++i) {
         const int qb = PER * tid + i;
@@ -348,9 +376,8 @@ struct ResTile {
             if (key != cur) {
               if (cur >= 0)
 #pragma unroll
-                for (int r = 0; r < NB; ++r) rw[at * NB + r] = y[r];
+                for (int r = 0; r < NB; ++r) rw[(tid + cur) * NB + r] = y[r];
               cur = key;
-              at = qb;
 #pragma unroll
               for (int r = 0; r < NB; ++r) y[r] = T(0);
             }
@@ -379,7 +406,7 @@ struct ResTile {
       }
       if (rows && cur >= 0)
 #pragma unroll
-        for (int r = 0; r < NB; ++r) rw[at * NB + r] = y[r];
+        for (int r = 0; r < NB; ++r) rw[(tid + cur) * NB + r] = y[r];
     };
 #pragma unroll
     for (int r = 0; r < NB; ++r) q[r] = T(0);
@@ -397,11 +424,9 @@ struct ResTile {
         q[0] = d[0] * xi[0] + d[2] * xi[1];
         q[1] = d[2] * xi[0] + d[1] * xi[1];
       }
-      // one piece per lane that owns blocks of the row, at its first of them
+      // one piece per lane that owns blocks of the row
       const int q0 = rps[tid], q1 = rps[tid + 1];
-      for (int p = q0; p < q1; p = (p / PER + 1) * PER)
-#pragma unroll
-        for (int r = 0; r < NB; ++r) q[r] += rw[p * NB + r];
+      if (q0 < q1) add_run(rw, tid + q0 / PER, tid + (q1 - 1) / PER + 1, q);
     };
     if constexpr (ONE) {
       blocks(true, false);
@@ -470,22 +495,33 @@ struct ResTile {
     return true;
   }
 
+  // Empties the tile's row nodes of the vector z and the partials it sent: the
+  // side that wrote them does, whose words are one run each, so that a store
+  // instruction fills whole lines (a reader would empty them a node at a time;
+  // every request of a line costs the fabric about the same).
+  __device__ __forceinline__ void empty_rows(double* z) const {
+    for (int e = lane_of_tile(lane); e < nr * NB; e += 256)
+      peer_empty(at_byte(z, 8u * (uint32_t)(NB * I0 + e)));
+  }
+  __device__ __forceinline__ void empty_partials(T* epart) const {
+    for (int e = lane_of_tile(lane); e < (ncols - nr) * NB; e += 256)
+      peer_empty(at_byte(epart, (uint32_t)sizeof(T) * (uint32_t)(NB * ext0 + e)));
+  }
+
   // The partials of the tile's row nodes.  look() fetches the lane's words,
   // kMerge at a time, into LDS (buffers of the product, free by then) as they
-  // arrive and empties them for the next but one product of the tiles that
-  // send them; it is called until it returns true (e: the lane's next word).
+  // arrive; it is called until it returns true (e: the lane's next word).
   // After a barrier add() adds the row node's partials to q in list order.
   __device__ __forceinline__ bool look(T* epart, int& e) const {
     while (e < nm) {
-      uint32_t off[kMerge];
       peer_w<T> w[kMerge];
       bool ok = true;
 #pragma unroll
       for (int j = 0; j < kMerge; ++j)
         if (e + 256 * j < nm) {
           const int k = (e + 256 * j) / NB;
-          off[j] = (uint32_t)sizeof(T) * (uint32_t)(NB * mls[k] + (e + 256 * j - NB * k));
-          w[j] = peer_get(at_byte(epart, off[j]));
+          w[j] = peer_get(at_byte(
+              epart, (uint32_t)sizeof(T) * (uint32_t)(NB * mls[k] + (e + 256 * j - NB * k))));
         }
 #pragma unroll
       for (int j = 0; j < kMerge; ++j)
@@ -495,7 +531,6 @@ struct ResTile {
       for (int j = 0; j < kMerge; ++j)
         if (e + 256 * j < nm) {
           tr[e + 256 * j] = PeerWord<T>::value(w[j]);
-          peer_empty(at_byte(epart, off[j]));
         }
       e += 256 * kMerge;
     }

@@ -1213,10 +1213,8 @@ extern "C" int elastic_time_assembly(elastic_ctx* xc, int32_t reps, double* ms) 
 // return with its consistent tangent (Simo & Hughes 1998, Box 3.2).  The
 // reference reaches no plasticity from its driver, so there is no reference
 // result to match; Voigt order xx, yy, zz, xy, yz, zx, engineering shears.
-// One 64-lane wavefront per element of a colour: lanes 0..7 integrate the 8
-// Gauss points (same points, shape functions and Jacobian as elmt07_mec),
-// then all lanes form K_t = sum B^T C B det and f = sum B^T sigma det, and the
-// element is added to ad/al and b (b -= f) through the slot map.
+// The Gauss points, shape functions and Jacobian are elmt07_mec's; K_t = sum
+// B^T C B det and b -= f = sum B^T sigma det, added through the slot map.
 namespace elastic {
 
 struct J2Dev {
@@ -1270,42 +1268,57 @@ __device__ inline void j2_point(const double* eps, const double* epn, double aln
     }
 }
 
-// B column of dof r of a node: rows and the derivative each row takes
-__device__ inline void bcol(int r, int* row, int* der) {
-  if (r == 0) row[0] = 0, der[0] = 0, row[1] = 3, der[1] = 1, row[2] = 5, der[2] = 2;
-  else if (r == 1) row[0] = 1, der[0] = 1, row[1] = 3, der[1] = 0, row[2] = 4, der[2] = 2;
-  else row[0] = 2, der[0] = 2, row[1] = 4, der[1] = 1, row[2] = 5, der[2] = 0;
+// kJ2E elements of a colour per 256-lane workgroup: 36 node pairs each fill its
+// lanes (252 of 256).  One lane per (element, Gauss point) forms the derivatives,
+// integrates the point and leaves det C (its 21 different entries) and det sigma
+// in LDS; one lane per dof forms f; one lane per node pair (na >= nb) forms the
+// 3x3 block of K_t from the B columns written out (every product with a zero of B
+// left out) and adds it through the slot map.  One 64-lane wavefront per element,
+// 8 of its lanes integrating and each then forming 9 entries by indexed B columns,
+// took 80 us per colour of hex8 36^3; this takes 37, about two thirds of it the
+// read-modify-writes of 24-byte runs of al (4 TB/s of whole lines).
+constexpr int kJ2E = 7;
+constexpr int kJ2Pairs = 36;
+// entry (r, c) of a symmetric 6x6 matrix stored by rows r <= c
+__host__ __device__ constexpr int sym6(int r, int c) {
+  return r <= c ? r * 6 - r * (r - 1) / 2 + (c - r) : sym6(c, r);
 }
 
-__global__ __launch_bounds__(64) void k_j2_hex8(AsmArgs a, J2Dev j, int c0, int lhs) {
-  constexpr int NEN = 8, NST = 24, NPAIR = NST * (NST + 1) / 2, NENT = NST * NST;
-  __shared__ double xl[NEN * 3], ul[NST], dX[8][3][NEN], Cg[8][36], Sg[8][6], s[NENT];
-  __shared__ int32_t ldv[NST];
-  __shared__ int bad;
-  const int el = a.order[c0 + blockIdx.x];
+__global__ __launch_bounds__(256) void k_j2_hex8(AsmArgs a, J2Dev j, int c0, int cnt, int lhs) {
+  constexpr int NEN = 8, NST = 24, NTRI = NST * (NST + 1) / 2;
+  __shared__ double xl[kJ2E][NST], ul[kJ2E][NST], dX[kJ2E][8][3][NEN];
+  __shared__ __align__(16) double Cg[kJ2E][8][22];
+  __shared__ double Sg[kJ2E][8][6];
+  __shared__ int32_t ldv[kJ2E][NST], elno[kJ2E], mat[kJ2E], bad[kJ2E];
   const int tid = threadIdx.x;
-  const int32_t* ixe = a.ix + (size_t)el * (NEN + 1);
-  if (tid == 0) bad = 0;
-  if (tid < NEN * 3) xl[tid] = a.x[(size_t)(ixe[tid / 3] - 1) * 3 + tid % 3];
-  if (tid < NST) {
-    const size_t g = (size_t)(ixe[tid / 3] - 1) * 3 + tid % 3;
-    ldv[tid] = a.id[g];
-    ul[tid] = j.u[g];
+  const int e0 = blockIdx.x * kJ2E, ne = min(kJ2E, cnt - e0);
+  if (tid < ne * NST) {
+    const int e = tid / NST, k = tid - e * NST;
+    const int el = a.order[c0 + e0 + e];
+    const int32_t* ixe = a.ix + (size_t)el * (NEN + 1);
+    const size_t g = (size_t)(ixe[k / 3] - 1) * 3 + k % 3;
+    xl[e][k] = a.x[g];
+    ul[e][k] = j.u[g];
+    ldv[e][k] = a.id[g];
+    if (k == 0) {
+      elno[e] = el;
+      mat[e] = ixe[NEN] - 1;
+      bad[e] = 0;
+    }
   }
-  const double* em = a.e + (size_t)(ixe[NEN] - 1) * 15;
-  const double E = em[0], nu = em[1];
   __syncthreads();
-  if (tid < 8) {
-    const int gp = tid, lx = gp & 1, ly = (gp >> 1) & 1, lz = gp >> 2;
+  if (tid < ne * 8) {
+    const int e = tid >> 3, gp = tid & 7, lx = gp & 1, ly = (gp >> 1) & 1, lz = gp >> 2;
     double h[NEN], hx[NEN], hy[NEN], hz[NEN], det;
     sfhexa8_d(kPG2[lx], kPG2[ly], kPG2[lz], h, hx, hy, hz);
-    if (!jacob3d_d(hx, hy, hz, xl, NEN, &det)) bad = 1;
+    if (!jacob3d_d(hx, hy, hz, xl[e], NEN, &det)) bad[e] = 1;
     double eps[6] = {0, 0, 0, 0, 0, 0};
+#pragma unroll
     for (int n = 0; n < NEN; ++n) {
-      dX[gp][0][n] = hx[n];
-      dX[gp][1][n] = hy[n];
-      dX[gp][2][n] = hz[n];
-      const double ux = ul[3 * n], uy = ul[3 * n + 1], uz = ul[3 * n + 2];
+      dX[e][gp][0][n] = hx[n];
+      dX[e][gp][1][n] = hy[n];
+      dX[e][gp][2][n] = hz[n];
+      const double ux = ul[e][3 * n], uy = ul[e][3 * n + 1], uz = ul[e][3 * n + 2];
       eps[0] += hx[n] * ux;
       eps[1] += hy[n] * uy;
       eps[2] += hz[n] * uz;
@@ -1313,62 +1326,86 @@ __global__ __launch_bounds__(64) void k_j2_hex8(AsmArgs a, J2Dev j, int c0, int 
       eps[4] += hz[n] * uy + hy[n] * uz;
       eps[5] += hz[n] * ux + hx[n] * uz;
     }
-    const size_t q = (size_t)el * 8 + gp;
+    const double* em = a.e + (size_t)mat[e] * 15;
+    const size_t q = (size_t)elno[e] * 8 + gp;
     double epn[6], sig[6], C[36], ep[6], al;
+#pragma unroll
     for (int k = 0; k < 6; ++k) epn[k] = j.ep_n[q * 6 + k];
-    j2_point(eps, epn, j.al_n[q], E, nu, j.sy, j.H, sig, C, ep, &al);
-    for (int k = 0; k < 6; ++k) Sg[gp][k] = sig[k] * det;
-    for (int k = 0; k < 36; ++k) Cg[gp][k] = C[k] * det;
-    for (int k = 0; k < 6; ++k) j.ep_t[q * 6 + k] = ep[k];
+    j2_point(eps, epn, j.al_n[q], em[0], em[1], j.sy, j.H, sig, C, ep, &al);
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+      Sg[e][gp][k] = sig[k] * det;
+      j.ep_t[q * 6 + k] = ep[k];
+    }
+#pragma unroll
+    for (int r = 0; r < 6; ++r)
+#pragma unroll
+      for (int c = r; c < 6; ++c) Cg[e][gp][sym6(r, c)] = C[r * 6 + c] * det;
     j.al_t[q] = al;
   }
   __syncthreads();
-  if (bad) {
-    if (tid == 0) a.err[0] = el + 1;
-    return;
-  }
-  // internal force, b -= f
-  if (tid < NST) {
-    const int n = tid / 3, r = tid % 3;
-    int row[3], der[3];
-    bcol(r, row, der);
-    double f = 0.0;
-    for (int gp = 0; gp < 8; ++gp)
-      for (int k = 0; k < 3; ++k) f += dX[gp][der[k]][n] * Sg[gp][row[k]];
-    const int k = ldv[tid];
-    if (k > 0 && k <= a.neq) a.b[k - 1] = a.b[k - 1] - f;
-  }
-  if (!lhs) return;
-  for (int en = tid; en < NENT; en += 64) {
-    const int i = en % NST, jj = en / NST;
-    const int na = i / 3, r = i % 3, nb = jj / 3, c = jj % 3;
-    int ri[3], di[3], rj[3], dj[3];
-    bcol(r, ri, di);
-    bcol(c, rj, dj);
-    double acc = 0.0;
-    for (int gp = 0; gp < 8; ++gp)
-      for (int p = 0; p < 3; ++p) {
-        const double bi = dX[gp][di[p]][na];
-        double t = 0.0;
-        for (int q2 = 0; q2 < 3; ++q2) t += Cg[gp][ri[p] * 6 + rj[q2]] * dX[gp][dj[q2]][nb];
-        acc += bi * t;
+  if (tid < ne && bad[tid]) a.err[0] = elno[tid] + 1;  // any offending element is reported
+  if (tid < ne * NST) {  // internal force, b -= f
+    const int e = tid / NST, k = tid - e * NST, n = k / 3, r = k - 3 * n;
+    const int eq = ldv[e][k];
+    if (!bad[e] && eq > 0 && eq <= a.neq) {
+      // rows of the B column of dof r, with the derivative each takes
+      const int k1 = r == 2 ? 4 : 3, k2 = r == 1 ? 4 : 5;
+      const int d1 = r == 0 ? 1 : r == 1 ? 0 : 1, d2 = r == 2 ? 0 : 2;
+      double f = 0.0;
+      for (int gp = 0; gp < 8; ++gp) {
+        f += dX[e][gp][r][n] * Sg[e][gp][r];
+        f += dX[e][gp][d1][n] * Sg[e][gp][k1];
+        f += dX[e][gp][d2][n] * Sg[e][gp][k2];
       }
-    s[en] = acc;  // s(i,j) at i + NST*j
+      a.b[eq - 1] = a.b[eq - 1] - f;
+    }
   }
-  __syncthreads();
-  const int32_t* sl = a.slots + (size_t)el * NPAIR;
-  for (int pp = tid; pp < NPAIR; pp += 64) {
-    const int32_t t = sl[pp];
-    if (t == -1) continue;
-    int i = (int)((sqrtf(8.0f * pp + 1.0f) - 1.0f) * 0.5f);
-    while ((i + 1) * (i + 2) / 2 <= pp) ++i;
-    while (i * (i + 1) / 2 > pp) --i;
-    const int jx = pp - i * (i + 1) / 2;
-    if (t <= -2) {
-      const int k = -t - 2;
-      a.ad[k] = a.ad[k] + s[i * NST + i];
-    } else {
-      a.al[t] = a.al[t] + (ldv[i] > ldv[jx] ? s[jx * NST + i] : s[i * NST + jx]);
+  if (!lhs || tid >= ne * kJ2Pairs) return;
+  const int e = tid / kJ2Pairs, pr = tid - e * kJ2Pairs;  // pr = na(na+1)/2 + nb
+  if (bad[e]) return;
+  int na = 0;
+#pragma unroll
+  for (int k = 1; k < NEN; ++k) na += pr >= k * (k + 1) / 2;
+  const int nb = pr - na * (na + 1) / 2;
+  double acc[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
+  for (int gp = 0; gp < 8; ++gp) {
+#pragma clang fp contract(fast)  // (no reference order to keep here)
+    const double xa = dX[e][gp][0][na], ya = dX[e][gp][1][na], za = dX[e][gp][2][na];
+    const double xb = dX[e][gp][0][nb], yb = dX[e][gp][1][nb], zb = dX[e][gp][2][nb];
+    const double* C = Cg[e][gp];
+    double t[6][3];
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+      const double s0 = C[sym6(k, 0)], s1 = C[sym6(k, 1)], s2 = C[sym6(k, 2)];
+      const double s3 = C[sym6(k, 3)], s4 = C[sym6(k, 4)], s5 = C[sym6(k, 5)];
+      t[k][0] = s0 * xb + s3 * yb + s5 * zb;
+      t[k][1] = s1 * yb + s3 * xb + s4 * zb;
+      t[k][2] = s2 * zb + s4 * yb + s5 * xb;
+    }
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      acc[0][c] += xa * t[0][c] + ya * t[3][c] + za * t[5][c];
+      acc[1][c] += ya * t[1][c] + xa * t[3][c] + za * t[4][c];
+      acc[2][c] += za * t[2][c] + ya * t[4][c] + xa * t[5][c];
+    }
+  }
+  const int32_t* sl = a.slots + (size_t)elno[e] * NTRI;
+  int32_t t[3][3];
+#pragma unroll
+  for (int r = 0; r < 3; ++r) {
+    const int i = 3 * na + r;
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+      t[r][c] = na == nb && c > r ? -1 : sl[i * (i + 1) / 2 + 3 * nb + c];
+  }
+#pragma unroll
+  for (int r = 0; r < 3; ++r) {
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      if (t[r][c] == -1) continue;
+      double* at = t[r][c] <= -2 ? a.ad + (-t[r][c] - 2) : a.al + t[r][c];
+      *at = *at + acc[r][c];
     }
   }
 }
@@ -1525,7 +1562,9 @@ extern "C" int elastic_j2_assemble(elastic_ctx* xc, int32_t lhs, double* rnorm) 
   }
   for (int k = 0; k < m->ncolors; ++k) {
     const int c0 = m->color_start[k], cnt = m->color_start[k + 1] - c0;
-    if (cnt > 0) hipLaunchKernelGGL(k_j2_hex8, dim3(cnt), dim3(64), 0, s, a, d, c0, lhs);
+    if (cnt > 0)
+      hipLaunchKernelGGL(k_j2_hex8, dim3((cnt + kJ2E - 1) / kJ2E), dim3(256), 0, s, a, d, c0, cnt,
+                         lhs);
   }
   int32_t err = 0;
   ELASTIC_HIP_CHECK(c, hipMemcpyAsync(&err, m->err, sizeof(int32_t), hipMemcpyDeviceToHost, s));

@@ -427,6 +427,13 @@ int pcg_resident_plan(Context* c, bool fp32_operator, bool bdiag, bool v32);
 int bicgstab_resident_plan(Context* c, bool bdiag);
 hipError_t bicgstab_resident_launch(Context* c, const double* bm, const double* rr, int maxit,
                                     int tpw);
+// gmres_resident.hip: the inner steps of one FP64 cycle of k steps; `words` holds
+// gm_resident_words(k)
+constexpr int kGmWords = 4 * 264;  // per sum of a step
+inline size_t gm_resident_words(int k) { return kGmWords * (size_t)(k + 1); }
+int gmres_resident_plan(Context* c, bool bdiag, int k);
+hipError_t gmres_resident_launch(Context* c, const double* bm, double* basis, double* H, double* e,
+                                 double* words, int k, double econv, int tpw);
 // doubles of Context::res_x for the layout just built (0: no resident solve)
 size_t resident_words(Context* c);
 hipError_t pcg_resident_launch(Context* c, const PcgVecs& V, bool fp32_operator, int maxit,

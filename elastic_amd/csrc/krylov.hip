@@ -508,7 +508,8 @@ int bicgstab_run(Context* c, bool bdiag, bool fp32_operator, double tol, int max
 // modified form's chain moved four vectors per basis vector.  On hex8 17^3
 // (16,524 equations, GMRES(50)) a step bound by the chain's launches and a host
 // read took 155 us; these passes take 36 us (product 6.7, w and h1 7.7, the two
-// updates 9.1 and 6.2, step 4.2): 132 -> 30.6 ms for 849 steps.
+// updates 9.1 and 6.2, step 4.2): 132 -> 30.6 ms for 849 steps.  FP64 cycles of
+// systems that fit on the chip run there (gmres_resident.hip).
 // Small arrays (column-major like the reference): h (k+1) x k, c(k), s(k),
 // e(k+1), y(k).
 
@@ -876,8 +877,8 @@ static void gm_lds(K* kernel, size_t bytes) {
                               160 * 1024);
 }
 
-int gmres_run(Context* c, bool bdiag, bool fp32_operator, double tol, int maxit, int k,
-              KrylovResult* out) {
+static int gmres_iterate(Context* c, bool bdiag, bool fp32_operator, double tol, int maxit, int k,
+                         KrylovResult* out, bool resident) {
   hipStream_t s = c->stream;
   const int n = c->neq;
   if (k < 1) k = 50;
@@ -888,9 +889,11 @@ int gmres_run(Context* c, bool bdiag, bool fp32_operator, double tol, int maxit,
     c->gm_basis = c->gm_small = nullptr;
     c->gm_k = 0;
     // the small arrays, then the workgroups' shares of two passes over the basis
+    // and the words of a cycle on the chip
     if (hipMalloc((void**)&c->gm_basis, sizeof(double) * (size_t)(k + 1) * n) != hipSuccess ||
         hipMalloc((void**)&c->gm_small,
-                  sizeof(double) * ((size_t)(k + 1) * k + 4 * k + 2 + 2 * (size_t)kGmBlocks * k)) !=
+                  sizeof(double) * ((size_t)(k + 1) * k + 4 * k + 2 + 2 * (size_t)kGmBlocks * k +
+                                    gm_resident_words(k))) !=
             hipSuccess) {
       (void)hipGetLastError();
       return set_error(c, ELASTIC_OOM, "GMRES basis of " + std::to_string(k + 1) + " vectors");
@@ -906,6 +909,8 @@ int gmres_run(Context* c, bool bdiag, bool fp32_operator, double tol, int maxit,
   double* S[2];  // the workgroups' shares: k rows of gg.blocks each
   S[0] = c->gm_small + (size_t)(k + 1) * k + 4 * k + 2;
   S[1] = S[0] + (size_t)kGmBlocks * k;
+  double* words = S[1] + (size_t)kGmBlocks * k;
+  const int tpw = resident && !fp32_operator ? gmres_resident_plan(c, bdiag, k) : 0;
   double *x = c->v64[VX], *b = c->v64[VB], *t = c->v64[VT], *u = c->v64[VU];
   const double* m = c->A64.m;
   const double* bm = bdiag ? solver_bm(c) : nullptr;
@@ -957,7 +962,12 @@ int gmres_run(Context* c, bool bdiag, bool fp32_operator, double tol, int maxit,
     }
     hipLaunchKernelGGL(k_gm_scale, G, TB, 0, s, n, g(1), (const double*)a.e);
     ++cycles;
-    for (int i = 1; i <= k; ++i) {
+    bool held = false;
+    if (tpw > 0) {
+      held = gmres_resident_launch(c, bm, c->gm_basis, a.h, a.e, words, k, econv, tpw) == hipSuccess;
+      if (!held) (void)hipGetLastError();  // not launched
+    }
+    for (int i = 1; i <= k && !held; ++i) {
       launch_spmv(c, op32, g(i), t, c->epart64, &sc->gm_done);
       const MergeArgs mg = merge_of(c, c->epart64, epart_f32(c, op32));
       if (bm) hipLaunchKernelGGL(k_gm_merge, G, TB, 0, s, n, mg, t, u);
@@ -1000,6 +1010,8 @@ int gmres_run(Context* c, bool bdiag, bool fp32_operator, double tol, int maxit,
                        (const double*)a.y, x, (const SolveScalars*)sc);
     rc = read_scalars();
     if (rc) return rc;
+    if (held && hs->lost)  // a workgroup did not arrive: start over with launches
+      return gmres_iterate(c, bdiag, fp32_operator, tol, maxit, k, out, false);
     nit += hs->gm_ni;
     if (!fp32_operator && hs->gm_e <= econv) conv = true;
   }
@@ -1021,6 +1033,11 @@ int gmres_run(Context* c, bool bdiag, bool fp32_operator, double tol, int maxit,
   out->done = conv;
   out->status = conv ? ELASTIC_OK : ELASTIC_MAXIT;
   return ELASTIC_OK;
+}
+
+int gmres_run(Context* c, bool bdiag, bool fp32_operator, double tol, int maxit, int k,
+              KrylovResult* out) {
+  return gmres_iterate(c, bdiag, fp32_operator, tol, maxit, k, out, true);
 }
 
 }  // namespace elastic

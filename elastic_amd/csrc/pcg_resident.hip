@@ -72,15 +72,21 @@ void resident_clear(Context* c, size_t t_size) {
                      t_size == 4 ? 2 * next : (int64_t)0, c->scal);
 }
 
-hipError_t resident_start(Context* c, const void* kernel, int tpw, size_t lds, void* args) {
+void resident_empty(Context* c, u64* words, int64_t n) {
+  hipLaunchKernelGGL(k_res_empty, dim3((unsigned)std::min<int64_t>((n + 255) / 256, 1024)),
+                     dim3(256), 0, c->stream, words, n, (uint32_t*)nullptr, (int64_t)0, c->scal);
+}
+
+hipError_t resident_start(Context* c, const void* kernel, int tpw, size_t lds, void* args,
+                          size_t fixed, int lanes) {
   if (lds > 65536) {
     const hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                             160 * 1024 - sizeof(ResShared) - 64);
+                                             160 * 1024 - sizeof(ResShared) - fixed - 64);
     if (e != hipSuccess) return e;
   }
   void* list[] = {args};
-  return hipLaunchCooperativeKernel(kernel, dim3((c->blk.ntiles + tpw - 1) / tpw), dim3(256 * tpw),
-                                    list, (unsigned)lds, c->stream);
+  return hipLaunchCooperativeKernel(kernel, dim3((c->blk.ntiles + tpw - 1) / tpw),
+                                    dim3(lanes ? lanes : 256 * tpw), list, (unsigned)lds, c->stream);
 }
 
 template <typename TV, typename T, typename VT, typename XT, int NB>

@@ -553,7 +553,12 @@ inline bool res_one_buffer(size_t t_size, int nblk_max, int tpw) {
 // empties every word of Context::res_x that a solve with sums of t_size bytes
 // exchanges, and the call's flags
 void resident_clear(Context* c, size_t t_size);
+// empties n more words
+void resident_empty(Context* c, u64* words, int64_t n);
 // raises the kernel's LDS limit where needed and launches it cooperatively
-hipError_t resident_start(Context* c, const void* kernel, int tpw, size_t lds, void* args);
+// (`fixed`: bytes of LDS the kernel declares beside ResShared; `lanes`: of a
+// workgroup, if not 256 per tile)
+hipError_t resident_start(Context* c, const void* kernel, int tpw, size_t lds, void* args,
+                          size_t fixed = 0, int lanes = 0);
 
 }  // namespace elastic

@@ -274,9 +274,10 @@ int elastic_set_tile_blocks(elastic_ctx* ctx, int32_t tile_blocks);
  * with HIP events on its stream -- a resident solve reads the device clock
  * around it on one workgroup; 0, the default: off),
  * "resident" (1, the default: PCG on systems that fit on the chip -- up to
- * 1,024 tiles; FP64 BiCGSTAB up to 512 -- runs its iterations in one cooperative
- * kernel that keeps the matrix in registers, and so does a batch; 0: one launch
- * per phase; both give the same method, their sums in different orders),
+ * 1,024 tiles; FP64 BiCGSTAB up to 512, FP64 GMRES up to 512 whose basis fits
+ * in LDS -- runs its iterations in one cooperative kernel that keeps the matrix
+ * in registers, and so does a batch; 0: one launch per phase; both give the same
+ * method, their sums in different orders),
  * "resident_looks" (how often a workgroup of such a kernel looks for a word of
  * another before it gives up and the solve starts over with launches),
  * "node_order" (1: the node-blocked tiles of a 3-dof layout are compact
@@ -318,9 +319,9 @@ int elastic_get_option(elastic_ctx* ctx, const char* name, int64_t* value);
  * the chip (option "resident") in one cooperative launch per step of
  * iters_per_step iterations, side by side; for the others every PCG phase is
  * one launch over all of them, and a step is captured once as a HIP graph
- * (use_graph != 0) and replayed while instances join and leave.  Each instance is a context holding its
- * structure, values (node-blocked layout) and b (elastic_upload_rhs); its
- * method is the PCG of elastic_solve (Iters.f:252-524, Jacobi), FP64 or
+ * (use_graph != 0) and replayed while instances join and leave.  Each
+ * instance is a context holding its structure, values (node-blocked layout)
+ * and b (elastic_upload_rhs); its method is the PCG of elastic_solve (Iters.f:252-524, Jacobi), FP64 or
  * MIXED, and its result is bit for bit the same alone and in any mix.  x is
  * left in the context (elastic_download_x).  One host thread drives a batch;
  * other threads may prepare contexts meanwhile. */

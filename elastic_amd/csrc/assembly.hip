@@ -702,6 +702,7 @@ struct MeshDev {
   // nodal stresses: (element, local node) pairs of every node in ascending
   // element order, and the buffers of the stress pass (allocated on first use)
   int32_t *inc_ptr = nullptr, *inc = nullptr;
+  hipStream_t copies = nullptr;  // brings b back while the new values are packed
   double *pl = nullptr, *tx = nullptr, *tx0 = nullptr;
 };
 
@@ -717,6 +718,7 @@ void free_mesh(MeshDev* m) {
                   m->inc_ptr, m->inc, m->pl, m->tx, m->tx0};
   for (void* p : ptrs)
     if (p) hipFree(p);
+  if (m->copies) hipStreamDestroy(m->copies);
   delete m;
 }
 
@@ -1031,7 +1033,8 @@ extern "C" int elastic_set_mesh(elastic_ctx* xc, int32_t nnode, int32_t numel, i
   chk(up(&m->lf, lv.data(), lv.size(), s));
   chk(up<double>(&m->u, nullptr, (size_t)nnode * ndf, s));
   chk(up<double>(&m->b, nullptr, (size_t)c->neq, s));
-  chk(up<int32_t>(&m->err, nullptr, 1, s));
+  chk(up<int32_t>(&m->err, nullptr, 2, s));
+  chk(hipStreamCreateWithFlags(&m->copies, hipStreamNonBlocking));
   {  // node -> (element, local node) in ascending element order (tform_mec's order)
     std::vector<int32_t> ptr((size_t)nnode + 1, 0), inc;
     for (int el = 0; el < numel; ++el)
@@ -1061,6 +1064,14 @@ extern "C" int elastic_set_mesh(elastic_ctx* xc, int32_t nnode, int32_t numel, i
   return ELASTIC_OK;
 }
 
+// first = max over the zero entries of neq - i (0: none), so that the first row
+// wins; reading ad back for this took 0.4 ms of an assembly of hex8 50^3
+__global__ __launch_bounds__(256) void k_zero_diag(int neq, const double* __restrict__ ad,
+                                                   int32_t* first) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < neq && ad[i] == 0.0) atomicMax(first, neq - i);
+}
+
 // Pform.f:1-254: isw 2 (lhs: K into ad/al; rhs: b -= K_e u_e) or isw 4 (loads
 // into b).  u is u(ndf,nnode) (may be NULL: zero); b is b(neq), in/out on the
 // host (may be NULL when rhs = 0).
@@ -1082,7 +1093,7 @@ extern "C" int elastic_assemble(elastic_ctx* xc, int32_t isw, int32_t lhs, int32
   }
   if (rhs)
     ELASTIC_HIP_CHECK(c, hipMemcpyAsync(m->b, b, sizeof(double) * c->neq, hipMemcpyHostToDevice, s));
-  ELASTIC_HIP_CHECK(c, hipMemsetAsync(m->err, 0, sizeof(int32_t), s));
+  ELASTIC_HIP_CHECK(c, hipMemsetAsync(m->err, 0, 2 * sizeof(int32_t), s));
   if (isw == 2) {
     if (lhs) {
       ELASTIC_HIP_CHECK(c, hipMemsetAsync(c->A64.ad, 0, sizeof(double) * c->neq, s));
@@ -1102,25 +1113,28 @@ extern "C" int elastic_assemble(elastic_ctx* xc, int32_t isw, int32_t lhs, int32
       default: launch_loads<K_HEX8>(a, m, s); break;
     }
   }
-  int32_t err = 0;
-  ELASTIC_HIP_CHECK(c, hipMemcpyAsync(&err, m->err, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-  if (rhs)
-    ELASTIC_HIP_CHECK(c, hipMemcpyAsync(b, m->b, sizeof(double) * c->neq, hipMemcpyDeviceToHost, s));
+  const bool values = isw == 2 && lhs;
+  if (values)
+    hipLaunchKernelGGL(k_zero_diag, dim3((c->neq + 255) / 256), dim3(256), 0, s, c->neq,
+                       (const double*)c->A64.ad, m->err + 1);
+  int32_t err[2] = {0, 0};
+  ELASTIC_HIP_CHECK(c, hipMemcpyAsync(err, m->err, sizeof(err), hipMemcpyDeviceToHost, s));
   ELASTIC_HIP_CHECK(c, hipStreamSynchronize(s));
   ELASTIC_HIP_CHECK(c, hipGetLastError());
-  if (err) return set_error(c, ELASTIC_NEG_JACOBIAN, "non-positive Jacobian in element " + std::to_string(err));
-  if (isw == 2 && lhs) {
+  if (values && !err[0]) {
     // derived arrays of the new values (Jacobi inverse, FP32 copies)
-    std::vector<double> ad(c->neq);
-    ELASTIC_HIP_CHECK(c, hipMemcpyAsync(ad.data(), c->A64.ad, sizeof(double) * c->neq, hipMemcpyDeviceToHost, s));
-    ELASTIC_HIP_CHECK(c, hipStreamSynchronize(s));
-    c->zero_diag_row = -1;
-    for (int i = 0; i < c->neq; ++i)
-      if (ad[i] == 0.0) {
-        c->zero_diag_row = i + 1;
-        break;
-      }
+    c->zero_diag_row = err[1] > 0 ? c->neq + 1 - err[1] : -1;
     derive_operator(c);
+  }
+  if (rhs) {
+    ELASTIC_HIP_CHECK(c, hipMemcpyAsync(b, m->b, sizeof(double) * c->neq, hipMemcpyDeviceToHost,
+                                        m->copies));
+    ELASTIC_HIP_CHECK(c, hipStreamSynchronize(m->copies));
+  }
+  if (err[0])
+    return set_error(c, ELASTIC_NEG_JACOBIAN,
+                     "non-positive Jacobian in element " + std::to_string(err[0]));
+  if (values) {
     ELASTIC_HIP_CHECK(c, hipStreamSynchronize(s));
     c->values_set = true;
     c->bdiag_set = false;

@@ -9,6 +9,7 @@ solves with host or resident vectors).
 from __future__ import annotations
 
 import ctypes as C
+import threading
 
 import numpy as np
 
@@ -175,12 +176,25 @@ def solv(neq, nad, ia, ja, ad, al, m, b, x, tol=1e-11, maxit=10000, ngram=50, un
     c = _default_ctx
     ia = np.ascontiguousarray(ia, np.int32)
     ja = np.ascontiguousarray(ja[:nad], np.int32)
-    # the structure is rebuilt whenever its contents change, not only its sizes
+    # the structure is rebuilt whenever its contents change, not only its sizes;
+    # a pattern of the last one's sizes is compared while the values go up (hex8
+    # 43^3: 2.2 ms beside 2.9), which are sent again should it differ
     key = getattr(c, "_solv_pattern", None)
-    if key is None or not (np.array_equal(key[0], ia) and np.array_equal(key[1], ja)):
+    if key is not None and len(key[0]) == len(ia) and len(key[1]) == len(ja):
+        same = []
+        t = threading.Thread(target=lambda: same.append(
+            np.array_equal(key[0], ia) and np.array_equal(key[1], ja)))
+        t.start()
+        try:
+            c.set_values(ad, al)
+        finally:
+            t.join()
+    else:
+        same = [False]
+    if not same[0]:
         c.set_structure(ia, ja)
         c._solv_pattern = (ia.copy(), ja.copy())
-    c.set_values(ad, al)
+        c.set_values(ad, al)
     m[:] = 1.0 / ad
     xs, st = c.solve(b, solver=solver, precond=precond, precision=precision, tol=tol, maxit=maxit,
                      ngram=ngram)

@@ -7,22 +7,24 @@
 // built once at set-up.
 //
 // Per call, on the caller's stream:
-//   1. column counts of the pattern (integer atomics into cnt, cleared first
+//   1. column counts of the pattern (integer atomics into cnt, one for the
+//      entries that three consecutive rows have at the same place; cleared first
 //      by a fill kernel; no hipMemsetAsync, so the call can be captured);
 //   2. colptr = exclusive scan of the counts (three launches: block scans,
 //      the scan of the block totals, the offsets);
-//   3. every stored entry placed in its column's list (integer atomics on a
-//      cursor copied from colptr; half a wavefront per row, so that a row's
-//      atomics are in flight together);
+//   3. every stored entry placed in its column's list (as many atomics on a
+//      cursor copied from colptr; 32 lanes per three rows, so that their atomics
+//      are in flight together);
 //   4. per row, one wavefront orders the column's list by CSRC position, so
 //      the order, and the FP64 result, never depend on the atomics, and adds
 //      y_i = ad_i x_i + row i in CSRC order + column i in ascending rows,
 //      bit-identical to matvec_csrcsym1.
-// On hex8 28^3 (neq 70,644, nad 2.6 M) a call takes 157 us: counts 27,
-// placement 54 (bound by its atomics; 178 with one lane per row), ordering and
-// product 70.  The last replaces an insertion sort of every list by one lane
-// (1,113 us: a serial chain of dependent global loads and stores) and a gather
-// product with one lane per row (98 us, uncoalesced); the call took 1,403 us.
+// On hex8 28^3 (neq 70,644, nad 2.6 M) a call takes 128 us: counts 16,
+// placement 35, ordering and product 69.  The first two are bound by their
+// atomics (26 and 54 with one atomic per entry; 178 with one lane per row).  The
+// last replaces an insertion sort of every list by one lane (1,113 us: a serial
+// chain of dependent global loads and stores) and a gather product with one lane
+// per row (98 us, uncoalesced); the call took 1,403 us.
 #include <mutex>
 
 #include "elastic_internal.h"
@@ -53,13 +55,53 @@ __global__ __launch_bounds__(256) void k_fill(int64_t n, int32_t* __restrict__ p
   for (int64_t i = blockIdx.x * 256ll + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) p[i] = v;
 }
 
-__global__ __launch_bounds__(256) void k_count_cols(int64_t nad, int n,
+// The entries of rows r = 3 g .. r + 2 by 32 lanes: f(r, c, j0, m, a, q) for every
+// column c[j0] at place q of these rows, which m rows j >= j0 have there (entry
+// a[j] + q).  The dofs of a node
+// have the same columns in the same places of their rows, so that one atomic serves
+// three entries; rows that do not match (other node sizes, restrained dofs)
+// take one each.  A column outside the system is dropped.
+template <typename F>
+__device__ __forceinline__ void row_triples(int n, const int32_t* __restrict__ ia,
+                                            const int32_t* __restrict__ ja, F f) {
+  const int sub = threadIdx.x & 31;
+  for (int64_t r = 3 * (blockIdx.x * 8ll + (threadIdx.x >> 5)); r < n;
+       r += 3 * (int64_t)gridDim.x * 8) {
+    int a[3], len[3], longest = 0;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      a[j] = r + j < n ? ia[r + j] - 1 : 0;
+      len[j] = r + j < n ? ia[r + j + 1] - 1 - a[j] : 0;
+      longest = max(longest, len[j]);
+    }
+    for (int q = sub; q < longest; q += 32) {
+      int c[3];
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        c[j] = q < len[j] ? ja[a[j] + q] - 1 : -1;
+        if (c[j] >= n) c[j] = -1;
+      }
+#pragma unroll
+      for (int j0 = 0; j0 < 3; ++j0) {
+        bool seen = c[j0] < 0;
+        int m = 0;
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+          seen |= j < j0 && c[j] == c[j0];
+          m += j >= j0 && c[j] == c[j0];
+        }
+        if (!seen) f(r, c, j0, m, a, q);
+      }
+    }
+  }
+}
+
+__global__ __launch_bounds__(256) void k_count_cols(int n, const int32_t* __restrict__ ia,
                                                      const int32_t* __restrict__ ja,
                                                      int32_t* __restrict__ cnt) {
-  for (int64_t k = blockIdx.x * 256ll + threadIdx.x; k < nad; k += (int64_t)gridDim.x * 256) {
-    const int c = ja[k] - 1;
-    if (c >= 0 && c < n) atomicAdd(&cnt[c], 1);  // a column outside the system is dropped
-  }
+  row_triples(n, ia, ja, [&](int64_t, const int (&c)[3], int j0, int m, const int (&)[3], int) {
+    atomicAdd(&cnt[c[j0]], m);
+  });
 }
 
 // exclusive scan of in[0..n) into out[0..n), one kScanBlock chunk per
@@ -131,24 +173,23 @@ __global__ __launch_bounds__(256) void k_scan_add(int n, int32_t* __restrict__ c
   if (i == n) colptr[n] = tot[nb];
 }
 
-// every stored entry into its column's list (any order inside a list); 32
-// lanes per row
+// every stored entry into its column's list (any order inside a list)
 __global__ __launch_bounds__(256) void k_place(int n, const int32_t* __restrict__ ia,
                                                 const int32_t* __restrict__ ja,
                                                 int32_t* __restrict__ cursor,
                                                 int32_t* __restrict__ colk,
                                                 int32_t* __restrict__ colrow) {
-  const int sub = threadIdx.x & 31;
-  for (int64_t r = blockIdx.x * 8ll + (threadIdx.x >> 5); r < n; r += (int64_t)gridDim.x * 8) {
-    const int k2 = ia[r + 1] - 1;
-    for (int k = ia[r] - 1 + sub; k < k2; k += 32) {
-      const int c = ja[k] - 1;
-      if (c < 0 || c >= n) continue;  // as in the count
-      const int p = atomicAdd(&cursor[c], 1);
-      colk[p] = k;
-      colrow[p] = (int)r;
-    }
-  }
+  row_triples(n, ia, ja,
+              [&](int64_t r, const int (&c)[3], int j0, int m, const int (&a)[3], int q) {
+                int p = atomicAdd(&cursor[c[j0]], m);
+#pragma unroll
+                for (int j = 0; j < 3; ++j)
+                  if (j >= j0 && c[j] == c[j0]) {
+                    colk[p] = a[j] + q;
+                    colrow[p] = (int)r + j;
+                    ++p;
+                  }
+              });
 }
 
 // The list colk[a..b) ordered in place by one wavefront, with its rows
@@ -329,15 +370,16 @@ extern "C" int elastic_spmv_csrc_noalloc(int32_t neq, int64_t nad, const int32_t
   const int nb = (neq + kScanBlock - 1) / kScanBlock;
   hipLaunchKernelGGL(k_fill, dim3(grid_of(neq)), dim3(256), 0, s, (int64_t)neq, cnt, 0);
   if (nad > 0)
-    hipLaunchKernelGGL(k_count_cols, dim3(grid_of(nad)), dim3(256), 0, s, nad, (int)neq, ja, cnt);
+    hipLaunchKernelGGL(k_count_cols, dim3(grid_of(32 * (int64_t)(neq / 3 + 1))), dim3(256), 0, s,
+                       (int)neq, ia, ja, cnt);
   hipLaunchKernelGGL(k_scan_blocks, dim3(nb), dim3(256), 0, s, neq, (const int32_t*)cnt, colptr,
                      tot);
   hipLaunchKernelGGL(k_scan_totals, dim3(1), dim3(256), 0, s, nb, tot);
   hipLaunchKernelGGL(k_scan_add, dim3((neq + 1 + 255) / 256), dim3(256), 0, s, neq, colptr,
                      (const int32_t*)tot, nb, cnt);
   if (nad > 0) {
-    hipLaunchKernelGGL(k_place, dim3(grid_of(32 * (int64_t)neq)), dim3(256), 0, s, neq, ia, ja,
-                       cnt, colk, colrow);
+    hipLaunchKernelGGL(k_place, dim3(grid_of(32 * (int64_t)(neq / 3 + 1))), dim3(256), 0, s, neq,
+                       ia, ja, cnt, colk, colrow);
   }
   hipLaunchKernelGGL(k_sort_gather, dim3(grid_of(8 * (int64_t)neq)), dim3(256), 0, s, neq, ia, ja,
                      ad, al, (const int32_t*)colptr, colk, colrow, x, y);

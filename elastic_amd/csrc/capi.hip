@@ -835,9 +835,8 @@ static int post_stats(Context* c, elastic_stats* st, double* bnorm2, double* bno
 }
 
 void derive_operator(Context* c) {
-  if (c->blk.d2r) launch_recip_layout(c);  // m in the layout's node order
-  else launch_recip<double>(c->neq, c->A64.ad, c->A64.m, c->stream);
   if (c->layout_nb == 1) {
+    launch_recip<double>(c->neq, c->A64.ad, c->A64.m, c->stream);
     launch_cast<double, float>(c->neq, c->A64.ad, c->A32.ad, c->stream);
     launch_cast<double, float>(c->nad, c->A64.al, c->A32.al, c->stream);
   } else {

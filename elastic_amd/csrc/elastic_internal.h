@@ -391,8 +391,6 @@ void launch_spmv(Context* c, bool fp32, const double* x, double* y, double* epar
 // it stages it, i.e. the product of x + dx)
 // gathers the CSRC values into the node-blocked planes (after every assembly)
 void launch_block_pack(Context* c);
-// the Jacobi scale 1/ad in the compact layout order (into A64.m)
-void launch_recip_layout(Context* c);
 // vectors between the CSRC order and the compact layout order:
 //   to_layout: dst[nb*d + r] = src[nb*d2r[d] + r];  else the inverse
 void launch_permute(int nn, int nb, const int32_t* d2r, const double* src, double* dst,

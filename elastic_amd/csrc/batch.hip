@@ -1053,6 +1053,16 @@ static int pack_resident(elastic_batch* b) {
   return ELASTIC_OK;
 }
 
+// x = 0 and the method's start
+static void start_instance(elastic_batch* b, int k) {
+  const auto& S = b->slots[k];
+  hipLaunchKernelGGL(k_bt_init, dim3(S.nch), dim3(kThreads), 0, b->stream, b->d_insts, k);
+  hipLaunchKernelGGL(k_bt_init2, dim3(1), dim3(kThreads), 0, b->stream, b->d_insts, k, S.tol,
+                     S.maxit, b->delta);
+  if (S.res >= 0)
+    hipLaunchKernelGGL(k_bt_res_empty, dim3(256), dim3(256), 0, b->stream, b->d_insts, k);
+}
+
 // the step of the instances held on the chip, then the true residuals they
 // stopped for
 static int step_resident(elastic_batch* b) {
@@ -1060,14 +1070,22 @@ static int step_resident(elastic_batch* b) {
   for (const auto& L : b->res_launches) {
     const void* f = resident_kernel(L.variant);
     if (L.lds > 65536)
-      BATCH_HIP(b, hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       160 * 1024 - sizeof(ResShared) - 64));
+      (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                160 * 1024 - sizeof(ResShared) - 64);
     const BInst* insts = b->d_insts;
     const ResWg* wgs = b->d_rwgs + L.first;
     int passes = L.passes, iters = b->iters;
     void* args[] = {&insts, &wgs, &passes, &iters};
-    BATCH_HIP(b, hipLaunchCooperativeKernel(f, dim3(L.groups), dim3(256 * kResTiles), args,
-                                            (unsigned)L.lds, s));
+    if (hipLaunchCooperativeKernel(f, dim3(L.groups), dim3(256 * kResTiles), args, (unsigned)L.lds,
+                                   s) == hipSuccess)
+      continue;
+    (void)hipGetLastError();  // not launched: its instances start over on the lists
+    for (int k = 0; k < b->max_slots; ++k)
+      if (b->slots[k].used && b->slots[k].res == L.variant) {
+        b->slots[k].res = -1;
+        start_instance(b, k);
+        b->dirty = true;
+      }
   }
   if (!b->res_mixed) return ELASTIC_OK;
   int rc = set_lds_limit(b);
@@ -1190,16 +1208,6 @@ static int capture(elastic_batch* b) {
   for (int v = 0; v < kVariants; ++v) b->graph_sgrid[v] = b->sgrid[v];
   b->graph_vgrid = b->vgrid;
   return ELASTIC_OK;
-}
-
-// x = 0 and the method's start
-static void start_instance(elastic_batch* b, int k) {
-  const auto& S = b->slots[k];
-  hipLaunchKernelGGL(k_bt_init, dim3(S.nch), dim3(kThreads), 0, b->stream, b->d_insts, k);
-  hipLaunchKernelGGL(k_bt_init2, dim3(1), dim3(kThreads), 0, b->stream, b->d_insts, k, S.tol,
-                     S.maxit, b->delta);
-  if (S.res >= 0)
-    hipLaunchKernelGGL(k_bt_res_empty, dim3(256), dim3(256), 0, b->stream, b->d_insts, k);
 }
 
 // folds an instance's FP32 increments of x (no-op without them)

@@ -26,9 +26,11 @@
 // CU) iterate there (pcg_resident.h) instead of on the lists, side by side in one
 // cooperative launch per step and, when there are more than the chip holds, one
 // after the other, each system with exchange words of its own.  Per batch, lists
-// against resident: 16 plane sections of up to 160^2 elements 66.4 and 30.5 ms,
-// 8 hex8 12^3 7.7 and 3.5, 6 hex8 33^3 mixed 50.8 and 35.5, 8 hex8 40^3 mixed (each
-// fills the chip) 94.3 and 93.5.
+// against resident: 16 plane sections of up to 160^2 elements 66.4 and 29.2 ms,
+// 8 hex8 12^3 8.0 and 3.3, 6 hex8 33^3 mixed 50.8 and 31.8, 64 plane requests of up
+// to 512^2 (lists and chip together) 2,537 and 2,458.  Where every instance is large
+// (16 of 390 to 1,030 tiles, one or two on the chip at a time) the lists were 7%
+// faster, 418 against 449; an instance may not look at the others, so it stays.
 #include <algorithm>
 #include <chrono>
 #include <cmath>
@@ -887,11 +889,13 @@ struct elastic_batch {
   uint32_t* d_sw[kVariants] = {nullptr};
   size_t sw_cap[kVariants] = {0};
   uint32_t* d_vwork = nullptr;
-  // counts: the kVariants product lists, then vector items, then slots
+  // slots: all active ones, then (max_slots further on each) those on the lists
+  // and those on the chip; counts: the kVariants product lists, vector items, the
+  // three kinds of slots
   int32_t *d_slist = nullptr, *d_counts = nullptr;
   size_t vwork_cap = 0;
   std::vector<uint32_t> h_sw[kVariants], h_vwork;
-  std::vector<int32_t> h_slist, h_counts;
+  std::vector<int32_t> h_slist, h_llist, h_rlist, h_counts;
   // non-empty variant lists, + bit 8: mixed instances present, bits 9 / 10:
   // 2-D / 3-D mixed instances present (their device-built lists are served)
   unsigned mask = 0, graph_mask = ~0u;
@@ -913,6 +917,8 @@ struct elastic_batch {
   ResWg* d_rwgs = nullptr;
   size_t rwgs_cap = 0;
   unsigned res_mixed = 0;  // bits 9 / 10 as in mask
+  hipStream_t rstream = nullptr;  // the launches on the chip, beside the lists'
+  hipEvent_t fork = nullptr, join = nullptr;
   BStatus* h_status = nullptr;  // pinned: the kernel of the statuses writes it
   bool dirty = true, stepped = false;
   size_t lds = 0, graph_lds = 0;
@@ -951,18 +957,17 @@ static void launch_dyn_spmv(elastic_batch* b, int nb3, int mode) {
 }
 
 // true residuals where asked (instances at an even iteration); `mask`: bits 9 / 10
-static void replace_residuals(elastic_batch* b, unsigned mask) {
+static void replace_residuals(elastic_batch* b, unsigned mask, const int32_t* slots,
+                              const int32_t* scount) {
   hipStream_t s = b->stream;
   const dim3 TB(kThreads);
-  const int32_t* scount = b->d_counts + kVariants + 1;
-  hipLaunchKernelGGL(k_bt_dyn_list, dim3(1), dim3(256), 0, s, b->d_insts, b->d_slist, scount,
-                     b->d_dyn, 1);
+  hipLaunchKernelGGL(k_bt_dyn_list, dim3(1), dim3(256), 0, s, b->d_insts, slots, scount, b->d_dyn, 1);
   for (int nb3 = 0; nb3 < 2; ++nb3)
     if (mask & (nb3 ? 0x400u : 0x200u)) {
       launch_dyn_spmv(b, nb3, 1);
       hipLaunchKernelGGL(k_bt_dyn_resid, dim3(kDynGrid), TB, 0, s, b->d_insts, b->d_dyn, nb3);
     }
-  hipLaunchKernelGGL(k_bt_rel_finish, dim3(kMaxSlots), TB, 0, s, b->d_insts, b->d_slist, scount, 0);
+  hipLaunchKernelGGL(k_bt_rel_finish, dim3(kMaxSlots), TB, 0, s, b->d_insts, slots, scount, 0);
 }
 
 // one PCG iteration of every active instance; `it` is the iteration index in
@@ -972,7 +977,7 @@ static void enqueue_iteration(elastic_batch* b, int it) {
   const dim3 TB(kThreads);
   const int cur = it & 1;
   const int32_t* vcount = b->d_counts + kVariants;
-  const int32_t* scount = vcount + 1;
+  const int32_t *scount = vcount + 2, *slots = b->d_slist + b->max_slots;
   // mixed instances: FP64 products of those the progress guard handed over.
   // A hand-over happens only in the true-residual pass that ends odd
   // iterations, and a step starts at an even one, so the list is rebuilt on
@@ -981,7 +986,7 @@ static void enqueue_iteration(elastic_batch* b, int it) {
   const bool mixed = (b->mask & 0x100u) != 0;
   if (mixed) {
     if (cur == 0)
-      hipLaunchKernelGGL(k_bt_dyn_list, dim3(1), dim3(256), 0, s, b->d_insts, b->d_slist, scount,
+      hipLaunchKernelGGL(k_bt_dyn_list, dim3(1), dim3(256), 0, s, b->d_insts, slots, scount,
                          b->d_dyn, 0);
     for (int nb3 = 0; nb3 < 2; ++nb3)
       if (b->mask & (nb3 ? 0x400u : 0x200u))
@@ -991,13 +996,12 @@ static void enqueue_iteration(elastic_batch* b, int it) {
     if (b->mask & (1u << v))
       launch_variant(v, dim3(b->sgrid[v]), TB, variant_lds(b, v), s, b->d_insts, b->d_sw[v],
                      b->d_counts + v);
-  hipLaunchKernelGGL(k_bt_sum_shares, dim3(kMaxSlots), TB, 0, s, b->d_insts, b->d_slist, scount);
+  hipLaunchKernelGGL(k_bt_sum_shares, dim3(kMaxSlots), TB, 0, s, b->d_insts, slots, scount);
   hipLaunchKernelGGL(k_bt_update, dim3(b->vgrid), TB, 0, s, b->d_insts, b->d_vwork, vcount, cur);
   hipLaunchKernelGGL(k_bt_pupdate, dim3(b->vgrid), TB, 0, s, b->d_insts, b->d_vwork, vcount, cur);
-  if (cur == 1 && mixed) replace_residuals(b, b->mask);  // every second iteration
+  if (cur == 1 && mixed) replace_residuals(b, b->mask, slots, scount);  // every second iteration
 }
 
-static int set_lds_limit(elastic_batch* b);
 
 // Packs the instances held on the chip, one launch per variant and at most one
 // workgroup per CU, the largest first, into as few passes as hold them.
@@ -1063,10 +1067,8 @@ static void start_instance(elastic_batch* b, int k) {
     hipLaunchKernelGGL(k_bt_res_empty, dim3(256), dim3(256), 0, b->stream, b->d_insts, k);
 }
 
-// the step of the instances held on the chip, then the true residuals they
-// stopped for
-static int step_resident(elastic_batch* b) {
-  hipStream_t s = b->stream;
+// The step of the instances held on the chip, on `s`.
+static void step_resident(elastic_batch* b, hipStream_t s) {
   for (const auto& L : b->res_launches) {
     const void* f = resident_kernel(L.variant);
     if (L.lds > 65536)
@@ -1087,11 +1089,6 @@ static int step_resident(elastic_batch* b) {
         b->dirty = true;
       }
   }
-  if (!b->res_mixed) return ELASTIC_OK;
-  int rc = set_lds_limit(b);
-  if (rc) return rc;
-  replace_residuals(b, b->res_mixed);
-  return ELASTIC_OK;
 }
 
 static int set_lds_limit(elastic_batch* b) {
@@ -1111,6 +1108,8 @@ static int upload_lists(elastic_batch* b) {
   for (auto& l : b->h_sw) l.clear();
   b->h_vwork.clear();
   b->h_slist.clear();
+  b->h_llist.clear();
+  b->h_rlist.clear();
   size_t lds = 0;
   bool mixed = false;
   unsigned mixed_nb = 0;
@@ -1120,6 +1119,7 @@ static int upload_lists(elastic_batch* b) {
     const BInst& I = b->h_insts[k];
     b->h_slist.push_back(k);
     lds = std::max(lds, S.lds);
+    (S.res >= 0 ? b->h_rlist : b->h_llist).push_back(k);
     if (S.res >= 0) continue;
     const int v0 = I.nb == 3 ? 3 : 0;
     // FP64 instances on the FP64 list; mixed ones on an FP32 list (their FP64
@@ -1165,10 +1165,12 @@ static int upload_lists(elastic_batch* b) {
   if (rc) return rc;
   rc = grow(b->d_vwork, b->vwork_cap, b->h_vwork.size());
   if (rc) return rc;
-  b->h_counts.assign(kVariants + 2, 0);
+  b->h_counts.assign(kVariants + 4, 0);
   for (int v = 0; v < kVariants; ++v) b->h_counts[v] = (int32_t)b->h_sw[v].size();
   b->h_counts[kVariants] = (int32_t)b->h_vwork.size();
   b->h_counts[kVariants + 1] = (int32_t)b->h_slist.size();
+  b->h_counts[kVariants + 2] = (int32_t)b->h_llist.size();
+  b->h_counts[kVariants + 3] = (int32_t)b->h_rlist.size();
   hipStream_t s = b->stream;
   for (int v = 0; v < kVariants; ++v)
     if (!b->h_sw[v].empty())
@@ -1177,9 +1179,12 @@ static int upload_lists(elastic_batch* b) {
   if (!b->h_vwork.empty())
     BATCH_HIP(b, hipMemcpyAsync(b->d_vwork, b->h_vwork.data(), b->h_vwork.size() * 4,
                                 hipMemcpyHostToDevice, s));
-  if (!b->h_slist.empty())
-    BATCH_HIP(b, hipMemcpyAsync(b->d_slist, b->h_slist.data(), b->h_slist.size() * 4,
-                                hipMemcpyHostToDevice, s));
+  int32_t* at = b->d_slist;
+  for (const auto* l : {&b->h_slist, &b->h_llist, &b->h_rlist}) {
+    if (!l->empty())
+      BATCH_HIP(b, hipMemcpyAsync(at, l->data(), l->size() * 4, hipMemcpyHostToDevice, s));
+    at += b->max_slots;
+  }
   BATCH_HIP(b, hipMemcpyAsync(b->d_counts, b->h_counts.data(), b->h_counts.size() * 4,
                               hipMemcpyHostToDevice, s));
   rc = pack_resident(b);
@@ -1239,9 +1244,12 @@ int elastic_batch_create(elastic_batch** out, int32_t device, int32_t max_slots,
     b->ncu = 256;
   std::memset(b->h_insts.data(), 0, sizeof(BInst) * max_slots);
   if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess ||
+      hipStreamCreateWithFlags(&b->rstream, hipStreamNonBlocking) != hipSuccess ||
+      hipEventCreateWithFlags(&b->fork, hipEventDisableTiming) != hipSuccess ||
+      hipEventCreateWithFlags(&b->join, hipEventDisableTiming) != hipSuccess ||
       hipMalloc((void**)&b->d_insts, sizeof(BInst) * max_slots) != hipSuccess ||
-      hipMalloc((void**)&b->d_slist, sizeof(int32_t) * max_slots) != hipSuccess ||
-      hipMalloc((void**)&b->d_counts, sizeof(int32_t) * (kVariants + 2)) != hipSuccess ||
+      hipMalloc((void**)&b->d_slist, sizeof(int32_t) * 3 * max_slots) != hipSuccess ||
+      hipMalloc((void**)&b->d_counts, sizeof(int32_t) * (kVariants + 4)) != hipSuccess ||
       hipMalloc((void**)&b->d_dyn, sizeof(DynList) * kDynLists) != hipSuccess ||
       hipMemset(b->d_dyn, 0, sizeof(DynList) * kDynLists) != hipSuccess ||
       hipHostMalloc((void**)&b->h_status, sizeof(BStatus) * max_slots) != hipSuccess) {
@@ -1260,6 +1268,7 @@ int elastic_batch_create(elastic_batch** out, int32_t device, int32_t max_slots,
 int elastic_batch_destroy(elastic_batch* b) {
   if (!b) return ELASTIC_OK;
   hipSetDevice(b->device);
+  if (b->rstream) hipStreamSynchronize(b->rstream);
   if (b->stream) hipStreamSynchronize(b->stream);
   // contexts of instances never retired go back to the CSRC order (with the
   // x their iteration reached)
@@ -1279,6 +1288,9 @@ int elastic_batch_destroy(elastic_batch* b) {
   for (uint32_t* p : b->d_sw)
     if (p) hipFree(p);
   if (b->h_status) hipHostFree(b->h_status);
+  if (b->rstream) hipStreamDestroy(b->rstream);
+  if (b->fork) hipEventDestroy(b->fork);
+  if (b->join) hipEventDestroy(b->join);
   if (b->stream) hipStreamDestroy(b->stream);
   delete b;
   return ELASTIC_OK;
@@ -1407,24 +1419,36 @@ int elastic_batch_step(elastic_batch* b) {
     if (rc) return rc;
   }
   if (b->h_slist.empty()) return ELASTIC_OK;
-  if (!b->res_launches.empty()) {
-    int rc = step_resident(b);
-    if (rc) return rc;
-  }
-  if (b->vgrid == 0) {  // every instance is on the chip
-  } else if (b->use_graph) {
+  if (b->use_graph && b->vgrid > 0) {
     bool grids = b->vgrid != b->graph_vgrid;
     for (int v = 0; v < kVariants; ++v) grids |= (b->mask & (1u << v)) && b->sgrid[v] != b->graph_sgrid[v];
     if (!b->gexec || b->graph_lds < b->lds || b->graph_mask != b->mask || grids) {
       int rc = capture(b);
       if (rc) return rc;
     }
-    BATCH_HIP(b, hipGraphLaunch(b->gexec, b->stream));
-  } else {
+  } else if (b->vgrid > 0 || b->res_mixed) {
     int rc = set_lds_limit(b);
     if (rc) return rc;
+  }
+  // the launches on the chip run beside those of the lists, which leave CUs free
+  // when few large instances are left: one after the other such a step took the
+  // sum of both
+  const bool both = !b->res_launches.empty() && b->vgrid > 0;
+  if (both) {
+    BATCH_HIP(b, hipEventRecord(b->fork, b->stream));
+    BATCH_HIP(b, hipStreamWaitEvent(b->rstream, b->fork, 0));
+  }
+  step_resident(b, both ? b->rstream : b->stream);
+  if (both) BATCH_HIP(b, hipEventRecord(b->join, b->rstream));
+  if (b->vgrid == 0) {  // every instance is on the chip
+  } else if (b->use_graph) {
+    BATCH_HIP(b, hipGraphLaunch(b->gexec, b->stream));
+  } else {
     for (int it = 0; it < b->iters; ++it) enqueue_iteration(b, it);
   }
+  if (both) BATCH_HIP(b, hipStreamWaitEvent(b->stream, b->join, 0));
+  if (b->res_mixed)  // the true residuals they stopped for
+    replace_residuals(b, b->res_mixed, b->d_slist + 2 * b->max_slots, b->d_counts + kVariants + 3);
   hipLaunchKernelGGL(k_bt_status, dim3(1), dim3(256), 0, b->stream, b->d_insts, b->d_slist,
                      b->d_counts + kVariants + 1, b->h_status);
   b->stepped = true;

@@ -107,7 +107,7 @@ __device__ __forceinline__ bool gm_exchange(const ResGm& g, int np, int seq, con
     h[j] = PeerWord<double>::value(w);
   }
   __syncthreads();
-  // every workgroup has sent shares of this round, so it has the last round's sums
+  // every workgroup has sent shares of exchange seq, so it has the sums of seq - 1
   if (seq > 0) {
     for (int j = tid; j < K; j += 64 * NW) peer_empty(old + (size_t)j * kResGroups + bid);
     if (tid < kGmCopies)

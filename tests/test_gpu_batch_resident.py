@@ -109,3 +109,29 @@ def test_limit_of_iterations_and_lost_peers(precision):
         assert lists[k][1]["iters"] == lost[k][1]["iters"]
     for s in systems:
         s.ctx.close()
+
+
+@pytest.mark.parametrize("precision", [FP64, MIXED])
+@pytest.mark.parametrize("use_graph", [True, False])
+def test_lists_and_chip_in_one_batch(precision, use_graph):
+    """instances on the lists and on the chip in the same steps, whose launches
+    run beside each other: each gives its bits of a batch of its own"""
+    from elastic_amd.serving import Batch
+
+    systems = _systems("hex8", (9, 8, 7, 10, 6), {}) + _systems("tria3", (30, 20), {})
+    for k, s in enumerate(systems):
+        s.ctx.set_option("resident", k % 2)
+    alone = [_run([s], precision)[0] for s in systems]
+    out = {}
+    with Batch(0, max_slots=len(systems), iters_per_step=8, use_graph=use_graph) as b:
+        for k, s in enumerate(systems):
+            assert b.submit(s.ctx, precision, 1e-11, 20000, k)
+        for _ in range(2000):
+            b.step()
+            for k, st in b.poll():
+                out[k] = (systems[k].ctx.download_x(), st)
+            if len(out) == len(systems):
+                break
+    for k, s in enumerate(systems):
+        assert np.array_equal(out[k][0], alone[k][0]) and out[k][1]["iters"] == alone[k][1]["iters"]
+        s.ctx.close()

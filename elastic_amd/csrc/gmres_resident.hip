@@ -56,7 +56,10 @@ static_assert(kResRounds * (kResGroups + kGmCopies) <= kGmWords, "words of an ex
 // k + 1 apart).  Sum j is formed by workgroup G - 1 - j (mod G; the first
 // workgroups are the slow ones) and fetched by everyone: all shares read by all
 // workgroups would be 6.4 MB per look for 126 of them and 50 sums.  Words are
-// emptied one round later and reused three rounds later, as in res_exchange.
+// emptied one round later and reused three rounds later, as in res_exchange: so
+// every workgroup drains its stores (peer_drain) between the round in which it
+// empties words and its shares two rounds on.  A step has two rounds and a drain
+// at its top; one that forms the norm again has three, and drains before the third.
 template <int TPW, int NW>
 __device__ __forceinline__ bool gm_exchange(const ResGm& g, int np, int seq, const double* dts,
                                             double* h, ResShared& sh) {
@@ -292,6 +295,7 @@ __global__ __launch_bounds__(gm_lanes<TPW>() * TPW) void k_gmres_resident(ResGm 
     for (int r = bl; r < R; r += WL) peer_put(zc + row0 + r, W[r]);
     if (!(n2 > 0.5 * ww)) {
       dots(i, i + 1);
+      peer_drain();  // (words emptied in the first round)
       __syncthreads();
       if (!gm_exchange<TPW, NW>(g, 1, seq++, dts, h, sh)) break;
       n2 = h[0];

@@ -179,7 +179,7 @@ def solv(neq, nad, ia, ja, ad, al, m, b, x, tol=1e-11, maxit=10000, ngram=50, un
     # the structure is rebuilt whenever its contents change, not only its sizes;
     # a pattern of the last one's sizes is compared while the values go up (hex8
     # 43^3: 2.2 ms beside 2.9), which are sent again should it differ
-    key = getattr(c, "_solv_pattern", None)
+    key = getattr(c, "_solv_pattern", None)  # None: the context holds no pattern of solv's
     if key is not None and len(key[0]) == len(ia) and len(key[1]) == len(ja):
         same = []
         t = threading.Thread(target=lambda: same.append(
@@ -192,6 +192,7 @@ def solv(neq, nad, ia, ja, ad, al, m, b, x, tol=1e-11, maxit=10000, ngram=50, un
     else:
         same = [False]
     if not same[0]:
+        c._solv_pattern = None  # (a pattern that is refused leaves the context without one)
         c.set_structure(ia, ja)
         c._solv_pattern = (ia.copy(), ja.copy())
         c.set_values(ad, al)

@@ -1,0 +1,64 @@
+"""solv compares the caller's pattern with the one its context holds.  A pattern
+that the library refuses leaves the context without any, so neither that pattern
+nor the one before it is the context's: the next call sets its structure first.
+The context is a stand-in that keeps the library's rules (values need a
+structure; a refused structure drops the one before)."""
+import numpy as np
+import pytest
+
+from elastic_amd import _lib, solver
+
+
+class _Held:
+    def __init__(self):
+        self.pattern, self.calls = None, []
+
+    def set_structure(self, ia, ja):
+        self.calls.append("structure")
+        self.pattern = None
+        if ja.size and ja.max() > len(ia) - 1:
+            raise _lib.ElasticError(_lib.BAD_ARG, "column outside the system")
+        self.pattern = (ia.copy(), ja.copy())
+
+    def set_values(self, ad, al):
+        self.calls.append("values")
+        if self.pattern is None:
+            raise _lib.ElasticError(_lib.NOT_READY, "structure not set")
+        self.used = (self.pattern[1].copy(), np.array(al))
+
+    def solve(self, b, **kw):
+        return np.array(b), {}
+
+
+PATTERNS = {"first": [1, 1, 2], "second": [1, 2, 3], "refused": [1, 2, 9], "longer": [1, 1, 2, 3]}
+
+
+def _call(name):
+    ja = np.array(PATTERNS[name], np.int32)
+    neq = 4
+    ia = np.array([1, 1, 2, 3, 1 + len(ja)], np.int32)
+    x = np.zeros(neq)
+    solver.solv(neq, len(ja), ia, ja, np.ones(neq), np.arange(1.0, 1 + len(ja)), np.zeros(neq),
+                np.ones(neq), x)
+    return ja
+
+
+@pytest.mark.parametrize("before", ["first", "longer"])
+@pytest.mark.parametrize("after", ["first", "second", "longer"])
+def test_a_refused_pattern_does_not_stand_in_the_way(monkeypatch, before, after):
+    c = _Held()
+    monkeypatch.setattr(solver, "_default_ctx", c)
+    _call(before)
+    with pytest.raises(_lib.ElasticError):
+        _call("refused")
+    ja = _call(after)
+    assert np.array_equal(c.used[0], ja) and len(c.used[1]) == len(ja)
+
+
+def test_patterns_of_the_same_sizes_are_told_apart(monkeypatch):
+    c = _Held()
+    monkeypatch.setattr(solver, "_default_ctx", c)
+    for name in ("first", "second", "second", "first"):
+        ja = _call(name)
+        assert np.array_equal(c.used[0], ja)
+    assert c.calls.count("structure") == 3

@@ -817,7 +817,7 @@ static size_t resident_lds(const Context* c, bool f32) {
 // the variant of an instance; -1: it iterates on the lists
 static int resident_variant(const Context* c, bool mixed, bool v32, int ncu) {
   const DevBlocks& b = c->blk;
-  if (!c->resident || !c->res_x || (mixed && c->accum32 && !v32)) return -1;
+  if (!resident_on(c) || (mixed && c->accum32 && !v32)) return -1;
   const bool f32 = mixed && c->accum32;
   if ((b.nb == 2 && f32) || (b.nblk_max > 512 && !f32)) return -1;
   if ((b.ntiles + kResTiles - 1) / kResTiles > std::min(ncu, kResGroups)) return -1;
@@ -877,6 +877,7 @@ struct elastic_batch {
     int ntiles = 0, nch = 0;
     size_t lds = 0;
     int res = -1;  // its variant on the chip (-1: it iterates on the lists)
+    int res_tiles = 0;  // tiles per workgroup of its iterations there
     double tol = 0.0;
     int maxit = 0;
     std::chrono::steady_clock::time_point t0;
@@ -1085,6 +1086,7 @@ static void step_resident(elastic_batch* b, hipStream_t s) {
     for (int k = 0; k < b->max_slots; ++k)
       if (b->slots[k].used && b->slots[k].res == L.variant) {
         b->slots[k].res = -1;
+        b->slots[k].res_tiles = 0;
         start_instance(b, k);
         b->dirty = true;
       }
@@ -1392,6 +1394,7 @@ int elastic_batch_submit(elastic_batch* b, elastic_ctx* x, int32_t precision, do
   S.maxit = maxit;
   S.nch = nch;
   S.res = res;
+  S.res_tiles = res >= 0 ? kResTiles : 0;
   start_instance(b, k);
   S.used = true;
   S.ctx = x;
@@ -1475,12 +1478,14 @@ int elastic_batch_poll(elastic_batch* b, int64_t* tags, elastic_stats* stats, in
       S.res = -1;
       b->dirty = true;
       if (st.lost) {
+        S.res_tiles = 0;
         start_instance(b, k);
         continue;
       }
     }
     if (!st.done) continue;
     tags[nd] = S.tag;
+    S.ctx->c.res_tiles = S.res_tiles;
     // an instance stopped by maxit still holds FP32 increments of x (a
     // converged one folded them at its last replacement)
     if (st.status != 0) {

@@ -234,7 +234,7 @@ __global__ __launch_bounds__(256 * TPW) void k_bicgstab_resident(ResBi g) {
 
 int bicgstab_resident_plan(Context* c, bool bdiag) {
   const DevBlocks& b = c->blk;
-  if (!c->res_x || !c->resident || (bdiag && b.nb != 3)) return 0;
+  if (!resident_on(c) || (bdiag && b.nb != 3)) return 0;
   // six vectors per row node beside the values: two tiles per CU at most
   return resident_tpw(c, 8, 2, sizeof(double) * b.nb * (size_t)b.ncols_max);
 }

@@ -605,8 +605,9 @@ int elastic_get_option(elastic_ctx* x, const char* name, int64_t* value) {
   else if (n == "tune_tiles") *value = c->tune_tiles ? 1 : 0;
   else if (n == "layout_nb") *value = c->gather ? 0 : c->layout_nb;
   else if (n == "node_order") *value = c->blk.d2r ? 1 : 0;
-  else if (n == "resident") *value = c->resident && c->res_x ? 1 : 0;
+  else if (n == "resident") *value = resident_on(c) ? 1 : 0;
   else if (n == "resident_looks") *value = c->resident_looks;
+  else if (n == "resident_tiles") *value = c->res_tiles;
   else return set_error((Context*)c, ELASTIC_BAD_ARG, "unknown option " + n);
   return ELASTIC_OK;
 }

@@ -244,6 +244,7 @@ struct Context {
   int ncu = 0;                // CUs of the device
   int clock_khz = 0;          // device clock of the resident products' timing
   bool resident = true;       // solves that fit on the chip run there
+  int res_tiles = 0;          // tiles per workgroup of the last solve on the chip (0: launches)
   int resident_looks = 1 << 22;  // looks at a peer's word before a wait is given up (~1 us each)
   // FP32 vectors of the mixed PCG with the FP32-sum operator (node-blocked):
   // p at p32, r at p32 + vec32_stride(neq), the Jacobi scale after that,
@@ -434,6 +435,8 @@ hipError_t gmres_resident_launch(Context* c, const double* bm, double* basis, do
                                  double* words, int k, double econv, int tpw);
 // doubles of Context::res_x for the layout just built (0: no resident solve)
 size_t resident_words(Context* c);
+// the layout has such words, and the context's solves may use them
+inline bool resident_on(const Context* c) { return c->resident && c->res_x; }
 hipError_t pcg_resident_launch(Context* c, const PcgVecs& V, bool fp32_operator, int maxit,
                                double* dslots, int tpw, float* p32, float* r32, float* m32,
                                float* dx32);

@@ -381,7 +381,7 @@ static int gm_room(const Context* c, int k, int tpw) {
 }
 
 int gmres_resident_plan(Context* c, bool bdiag, int k) {
-  if (!c->res_x || !c->resident || (bdiag && c->blk.nb != 3) || k > 256) return 0;
+  if (!resident_on(c) || (bdiag && c->blk.nb != 3) || k > 256) return 0;
   for (int tpw = 1; tpw <= 2; ++tpw)
     if ((c->blk.ntiles + tpw - 1) / tpw <= std::min(c->ncu, kResGroups) && gm_room(c, k, tpw))
       return tpw;

@@ -432,6 +432,7 @@ static int bicgstab_iterate(Context* c, bool bdiag, bool fp32_operator, double t
   bool op32 = fp32_operator;  // the progress guard may hand over to the FP64 operator
   // FP64 systems that fit on the chip iterate there, in one call
   const int tpw = resident && !reliable ? bicgstab_resident_plan(c, !jac) : 0;
+  c->res_tiles = 0;
   if (tpw > 0) {
     const hipError_t e = bicgstab_resident_launch(c, bm, rr, maxit, tpw);
     if (e == hipSuccess) {
@@ -440,6 +441,7 @@ static int bicgstab_iterate(Context* c, bool bdiag, bool fp32_operator, double t
       ELASTIC_HIP_CHECK(c, hipStreamSynchronize(s));
       if (c->scal_host->lost)  // a workgroup did not arrive: start over with launches
         return bicgstab_iterate(c, bdiag, fp32_operator, tol, maxit, delta, out, false);
+      c->res_tiles = tpw;
       it = maxit;
       done = c->scal_host->done != 0;
     } else {
@@ -911,6 +913,7 @@ static int gmres_iterate(Context* c, bool bdiag, bool fp32_operator, double tol,
   S[1] = S[0] + (size_t)kGmBlocks * k;
   double* words = S[1] + (size_t)kGmBlocks * k;
   const int tpw = resident && !fp32_operator ? gmres_resident_plan(c, bdiag, k) : 0;
+  c->res_tiles = 0;
   double *x = c->v64[VX], *b = c->v64[VB], *t = c->v64[VT], *u = c->v64[VU];
   const double* m = c->A64.m;
   const double* bm = bdiag ? solver_bm(c) : nullptr;
@@ -1012,6 +1015,7 @@ static int gmres_iterate(Context* c, bool bdiag, bool fp32_operator, double tol,
     if (rc) return rc;
     if (held && hs->lost)  // a workgroup did not arrive: start over with launches
       return gmres_iterate(c, bdiag, fp32_operator, tol, maxit, k, out, false);
+    if (held) c->res_tiles = tpw;
     nit += hs->gm_ni;
     if (!fp32_operator && hs->gm_e <= econv) conv = true;
   }

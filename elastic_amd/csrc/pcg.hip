@@ -655,6 +655,7 @@ static int pcg_iterate(Context* c, const PcgVecs& V, bool fp32_operator, double 
   // loop below starts an iteration from, so what it does not finish (the FP64
   // operator after a hand-over) goes on there.
   const int tpw = resident && tdots ? pcg_resident_plan(c, fp32_operator, !jac, v32) : 0;
+  c->res_tiles = 0;
   while (tpw > 0 && it < maxit && !done) {
     const hipError_t e = pcg_resident_launch(c, V, fp32_operator, maxit, dslots, tpw,
                                              v32 ? p32 : nullptr, r32, m32, dx32);
@@ -668,6 +669,7 @@ static int pcg_iterate(Context* c, const PcgVecs& V, bool fp32_operator, double 
     ELASTIC_HIP_CHECK(c, hipStreamSynchronize(s));
     if (c->scal_host->lost)  // a workgroup did not arrive: start over without the resident kernel
       return pcg_iterate(c, V, fp32_operator, tol, maxit, reliable, delta, dslots, false);
+    c->res_tiles = tpw;
     it = c->scal_host->iter;
     done = c->scal_host->done != 0;
     c->tprod_ms += (double)c->scal_host->prod_ticks / c->clock_khz;

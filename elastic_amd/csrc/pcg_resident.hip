@@ -125,7 +125,7 @@ static hipError_t res_run(Context* c, const PcgVecs& V, const TV* vals, const TV
 
 int pcg_resident_plan(Context* c, bool fp32_operator, bool bdiag, bool v32) {
   const DevBlocks& b = c->blk;
-  if (!c->res_x || !c->resident) return 0;
+  if (!resident_on(c)) return 0;
   if (bdiag && b.nb != 3) return 0;  // equation triples that are not nodes
   // FP32 sums: only with the FP32 vectors
   const bool f32 = fp32_operator && c->accum32;

@@ -274,10 +274,14 @@ int elastic_set_tile_blocks(elastic_ctx* ctx, int32_t tile_blocks);
  * with HIP events on its stream -- a resident solve reads the device clock
  * around it on one workgroup; 0, the default: off),
  * "resident" (1, the default: PCG on systems that fit on the chip -- up to
- * 1,024 tiles; FP64 BiCGSTAB up to 512, FP64 GMRES up to 512 whose basis fits
- * in LDS -- runs its iterations in one cooperative kernel that keeps the matrix
- * in registers, and so does a batch; 0: one launch per phase; both give the same
- * method, their sums in different orders),
+ * 1,024 tiles, FP32 sums and the block preconditioner in 3-D only; FP64 BiCGSTAB
+ * up to 512; FP64 GMRES up to 512 and cycles of at most 256 steps, where LDS
+ * holds the product's tile and at least half the cycle's basis (the rest is read
+ * from memory) -- runs its iterations in one cooperative kernel that keeps the
+ * matrix in registers; so does a batch for instances of up to 1,024 tiles, of at
+ * most 512 blocks if it sums in FP64, in 3-D with Jacobi if it sums in FP32; 0:
+ * one launch per phase; both give the same method, their sums in different
+ * orders),
  * "resident_looks" (how often a workgroup of such a kernel looks for a word of
  * another before it gives up and the solve starts over with launches),
  * "node_order" (1: the node-blocked tiles of a 3-dof layout are compact
@@ -310,7 +314,10 @@ int elastic_autotune(elastic_ctx* ctx, int32_t precision, int32_t reps, int32_t*
  * (lanes per tile of the FP64 / FP32-value product) or "layout_nb" (node
  * block size of the layout, 1 scalar rows, 0 the gather product);
  * "node_order" reads the order of the layout in use (1 compact), "resident"
- * whether solves that the method allows run on the chip. */
+ * whether the layout has the words that solves on the chip exchange (at least
+ * one of FP64 and FP32 sums fits) and they may be used; "resident_tiles": tiles
+ * per workgroup with which the last solve, or the last instance that left a batch,
+ * iterated on the chip (0: by launches, or started over with them). */
 int elastic_get_option(elastic_ctx* ctx, const char* name, int64_t* value);
 
 /* ------------------------------------------------------ batched serving */

@@ -921,6 +921,9 @@ struct elastic_batch {
   hipStream_t rstream = nullptr;  // the launches on the chip, beside the lists'
   hipEvent_t fork = nullptr, join = nullptr;
   BStatus* h_status = nullptr;  // pinned: the kernel of the statuses writes it
+  // an instance's workgroup gave up a wait: what is submitted from then on takes
+  // the lists (each could wait as long)
+  bool lost = false;
   bool dirty = true, stepped = false;
   size_t lds = 0, graph_lds = 0;
   hipGraphExec_t gexec = nullptr;
@@ -1378,7 +1381,7 @@ int elastic_batch_submit(elastic_batch* b, elastic_ctx* x, int32_t precision, do
   I.acc32 = c->accum32 ? 1 : 0;
   I.live = 1;
   I.ntiles = c->blk.ntiles;
-  const int res = resident_variant(c, I.fp32, v32, b->ncu);
+  const int res = b->lost ? -1 : resident_variant(c, I.fp32, v32, b->ncu);
   if (res >= 0) {
     I.res_x = c->res_x;
     I.res_next = c->blk.next_nodes * c->layout_nb;
@@ -1478,6 +1481,8 @@ int elastic_batch_poll(elastic_batch* b, int64_t* tags, elastic_stats* stats, in
       S.res = -1;
       b->dirty = true;
       if (st.lost) {
+        resident_gave_up(&S.ctx->c);
+        b->lost = true;
         S.res_tiles = 0;
         start_instance(b, k);
         continue;

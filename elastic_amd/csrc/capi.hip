@@ -267,6 +267,7 @@ static int build_layout(elastic_ctx* x) {
     nepart = (int64_t)nb * L.next_nodes;
     rc = rc ? rc : dalloc(c, &c->tdot, (size_t)L.ntiles);
     rc = rc ? rc : dalloc(c, &c->p32, 4 * vec32_stride(neq));
+    c->res_off = false;
     const size_t nres = resident_words(c);
     if (nres) rc = rc ? rc : dalloc(c, &c->res_x, nres);
   }
@@ -608,6 +609,7 @@ int elastic_get_option(elastic_ctx* x, const char* name, int64_t* value) {
   else if (n == "resident") *value = resident_on(c) ? 1 : 0;
   else if (n == "resident_looks") *value = c->resident_looks;
   else if (n == "resident_tiles") *value = c->res_tiles;
+  else if (n == "resident_lost") *value = c->res_lost;
   else return set_error((Context*)c, ELASTIC_BAD_ARG, "unknown option " + n);
   return ELASTIC_OK;
 }
@@ -642,6 +644,7 @@ int elastic_set_option(elastic_ctx* x, const char* name, int64_t value) {
     c->check_every = (int)value;
   } else if (n == "resident") {
     c->resident = value != 0;
+    c->res_off = false;
   } else if (n == "resident_looks") {
     if (value < 0 || value > (1 << 30)) return ELASTIC_BAD_ARG;
     c->resident_looks = (int)value;

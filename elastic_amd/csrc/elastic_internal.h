@@ -244,7 +244,9 @@ struct Context {
   int ncu = 0;                // CUs of the device
   int clock_khz = 0;          // device clock of the resident products' timing
   bool resident = true;       // solves that fit on the chip run there
+  bool res_off = false;       // not after one that gave up a wait (resident_gave_up)
   int res_tiles = 0;          // tiles per workgroup of the last solve on the chip (0: launches)
+  int64_t res_lost = 0;       // solves that gave up a wait and started over with launches
   int resident_looks = 1 << 22;  // looks at a peer's word before a wait is given up (~1 us each)
   // FP32 vectors of the mixed PCG with the FP32-sum operator (node-blocked):
   // p at p32, r at p32 + vec32_stride(neq), the Jacobi scale after that,
@@ -421,6 +423,15 @@ struct PcgVecs {
 // preconditioner does not allow it; a launch runs iterations until the solve
 // converges, asks for a true-residual replacement or reaches maxit.
 int pcg_resident_plan(Context* c, bool fp32_operator, bool bdiag, bool v32);
+// A workgroup of the context's solve did not see a peer's word in time: its solves
+// take the launches until the option "resident" is set or the layout built
+// again (whatever held the peer back may hold the next one back as long, seconds at the
+// default limit).
+inline void resident_gave_up(Context* c) {
+  c->res_off = true;
+  c->res_tiles = 0;
+  c->res_lost += 1;
+}
 // bicgstab_resident.hip: the FP64 iteration of bicgstab_run in one call, after
 // its initialisation; plan as above
 int bicgstab_resident_plan(Context* c, bool bdiag);
@@ -436,7 +447,7 @@ hipError_t gmres_resident_launch(Context* c, const double* bm, double* basis, do
 // doubles of Context::res_x for the layout just built (0: no resident solve)
 size_t resident_words(Context* c);
 // the layout has such words, and the context's solves may use them
-inline bool resident_on(const Context* c) { return c->resident && c->res_x; }
+inline bool resident_on(const Context* c) { return c->resident && !c->res_off && c->res_x; }
 hipError_t pcg_resident_launch(Context* c, const PcgVecs& V, bool fp32_operator, int maxit,
                                double* dslots, int tpw, float* p32, float* r32, float* m32,
                                float* dx32);

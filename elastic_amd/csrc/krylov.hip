@@ -439,8 +439,10 @@ static int bicgstab_iterate(Context* c, bool bdiag, bool fp32_operator, double t
       ELASTIC_HIP_CHECK(c, hipMemcpyAsync(c->scal_host, sc, sizeof(SolveScalars),
                                           hipMemcpyDeviceToHost, s));
       ELASTIC_HIP_CHECK(c, hipStreamSynchronize(s));
-      if (c->scal_host->lost)  // a workgroup did not arrive: start over with launches
+      if (c->scal_host->lost) {  // a workgroup did not arrive: start over with launches
+        resident_gave_up(c);
         return bicgstab_iterate(c, bdiag, fp32_operator, tol, maxit, delta, out, false);
+      }
       c->res_tiles = tpw;
       it = maxit;
       done = c->scal_host->done != 0;
@@ -1013,8 +1015,10 @@ static int gmres_iterate(Context* c, bool bdiag, bool fp32_operator, double tol,
                        (const double*)a.y, x, (const SolveScalars*)sc);
     rc = read_scalars();
     if (rc) return rc;
-    if (held && hs->lost)  // a workgroup did not arrive: start over with launches
+    if (held && hs->lost) {  // a workgroup did not arrive: start over with launches
+      resident_gave_up(c);
       return gmres_iterate(c, bdiag, fp32_operator, tol, maxit, k, out, false);
+    }
     if (held) c->res_tiles = tpw;
     nit += hs->gm_ni;
     if (!fp32_operator && hs->gm_e <= econv) conv = true;

@@ -667,8 +667,10 @@ static int pcg_iterate(Context* c, const PcgVecs& V, bool fp32_operator, double 
     ELASTIC_HIP_CHECK(c, hipMemcpyAsync(c->scal_host, sc, sizeof(SolveScalars),
                                         hipMemcpyDeviceToHost, s));
     ELASTIC_HIP_CHECK(c, hipStreamSynchronize(s));
-    if (c->scal_host->lost)  // a workgroup did not arrive: start over without the resident kernel
+    if (c->scal_host->lost) {  // a workgroup did not arrive: start over without the resident kernel
+      resident_gave_up(c);
       return pcg_iterate(c, V, fp32_operator, tol, maxit, reliable, delta, dslots, false);
+    }
     c->res_tiles = tpw;
     it = c->scal_host->iter;
     done = c->scal_host->done != 0;

@@ -283,7 +283,9 @@ int elastic_set_tile_blocks(elastic_ctx* ctx, int32_t tile_blocks);
  * one launch per phase; both give the same method, their sums in different
  * orders),
  * "resident_looks" (how often a workgroup of such a kernel looks for a word of
- * another before it gives up and the solve starts over with launches),
+ * another before it gives up and the solve starts over with launches; the
+ * context's solves, and instances submitted to that batch from then on, take the
+ * launches until "resident" is set or the layout built again),
  * "node_order" (1: the node-blocked tiles of a 3-dof layout are compact
  * breadth-first clusters of the node graph, in whose node order the solves
  * iterate -- b and x are exchanged with the caller in the CSRC order as
@@ -317,7 +319,8 @@ int elastic_autotune(elastic_ctx* ctx, int32_t precision, int32_t reps, int32_t*
  * whether the layout has the words that solves on the chip exchange (at least
  * one of FP64 and FP32 sums fits) and they may be used; "resident_tiles": tiles
  * per workgroup with which the last solve, or the last instance that left a batch,
- * iterated on the chip (0: by launches, or started over with them). */
+ * iterated on the chip (0: by launches, or started over with them);
+ * "resident_lost": solves and instances of this context that started over. */
 int elastic_get_option(elastic_ctx* ctx, const char* name, int64_t* value);
 
 /* ------------------------------------------------------ batched serving */

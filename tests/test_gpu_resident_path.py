@@ -39,7 +39,7 @@ def _system(kind, n, opts):
 def test_pcg(kind, n, opts, tpw):
     s = _system(kind, n, opts)
     three = kind in ("hex8", "tet4")
-    assert s.ctx.get_option("resident_tiles") == 0
+    assert s.ctx.get_option("resident_tiles") == s.ctx.get_option("resident_lost") == 0
     for precision, precond, sums32 in [(FP64, DIAG, 0), (FP64, BLOCKS, 0), (MIXED, DIAG, 0),
                                        (MIXED, BLOCKS, 0), (MIXED, DIAG, 1), (MIXED, BLOCKS, 1)]:
         want = tpw if three or (precond == DIAG and not (precision == MIXED and sums32)) else 0
@@ -49,6 +49,7 @@ def test_pcg(kind, n, opts, tpw):
             s.ctx.set_option("resident", resident)
             s.solve(precision=precision, precond=precond, tol=1e-8, maxit=20000)
             assert s.ctx.get_option("resident_tiles") == (want if resident else 0)
+    assert s.ctx.get_option("resident_lost") == 0
     s.ctx.close()
 
 
@@ -108,5 +109,68 @@ def test_batch(kind, n, opts, precision, tiles):
     a, b = _system(kind, n, opts), _system(kind, n, dict(opts, resident=0))
     print("path batch", kind, n, opts, precision, flush=True)
     assert _batch([a, b], precision) == [tiles, 0]
+    assert a.ctx.get_option("resident_lost") == 0
     a.ctx.close()
     b.ctx.close()
+
+
+@pytest.mark.parametrize("solver", ["pcg", "mixed", "bicgstab", "gmres", "batch"])
+def test_a_lost_solve_is_counted_and_not_repeated(solver):
+    """with no look left for its peers' words a solve is launched on the chip, gives
+    up and is counted; the next ones do not try again until the option is set, or a
+    layout built"""
+    from elastic_amd.solver import BICGSTAB, GMRES, PCG
+
+    s = _system("hex8", 12, {})
+
+    def solve():
+        if solver == "batch":
+            return _batch([s], FP64)[0]
+        s.solve(solver={"bicgstab": BICGSTAB, "gmres": GMRES}.get(solver, PCG), tol=1e-8,
+                precision=MIXED if solver == "mixed" else FP64)
+        return s.ctx.get_option("resident_tiles")
+
+    held = solve()
+    assert held > 0
+    looks = s.ctx.get_option("resident_looks")
+    s.ctx.set_option("resident_looks", 0)
+    for _ in range(2):
+        assert solve() == 0
+        assert s.ctx.get_option("resident_lost") == 1 and s.ctx.get_option("resident") == 0
+    s.ctx.set_option("resident_looks", looks)
+    assert solve() == 0
+    s.ctx.set_option("resident", 1)
+    assert solve() == held and s.ctx.get_option("resident_lost") == 1
+    s.ctx.set_option("resident_looks", 0)
+    assert solve() == 0 and s.ctx.get_option("resident_lost") == 2
+    s.ctx.set_option("resident_looks", looks)
+    s.ctx.set_structure(s.ia, s.ja)
+    ad, al = _system("hex8", 12, {}).values()
+    s.ctx.set_values(ad, al)
+    assert solve() == held
+    s.ctx.close()
+
+
+def test_a_batch_that_lost_an_instance_takes_the_lists():
+    """instances already on the chip stay there; later ones of the same batch go to
+    the lists, a new batch takes the chip again"""
+    from elastic_amd.serving import Batch
+
+    lost, beside, later = (_system("hex8", n, {}) for n in (8, 9, 7))
+    lost.ctx.set_option("resident_looks", 0)
+    for s in (lost, beside, later):
+        s.ctx.upload_rhs(s.b)
+    with Batch(0, max_slots=3, iters_per_step=8) as b:
+        assert b.submit(lost.ctx, FP64, 1e-9, 20000, 0) and b.submit(beside.ctx, FP64, 1e-9, 20000, 1)
+        b.step()
+        done = b.poll()
+        assert b.submit(later.ctx, FP64, 1e-9, 20000, 2)
+        while len(done) < 3:
+            b.step()
+            done += b.poll()
+    tiles = [s.ctx.get_option("resident_tiles") for s in (lost, beside, later)]
+    assert tiles == [0, 4, 0]
+    assert [s.ctx.get_option("resident_lost") for s in (lost, beside, later)] == [1, 0, 0]
+    assert _batch([later], FP64) == [4]
+    for s in (lost, beside, later):
+        s.ctx.close()

@@ -192,7 +192,7 @@ def solv(neq, nad, ia, ja, ad, al, m, b, x, tol=1e-11, maxit=10000, ngram=50, un
     else:
         same = [False]
     if not same[0]:
-        c._solv_pattern = None  # (a pattern that is refused leaves the context without one)
+        c._solv_pattern = None  # (a structure that fails may leave the context without one)
         c.set_structure(ia, ja)
         c._solv_pattern = (ia.copy(), ja.copy())
         c.set_values(ad, al)

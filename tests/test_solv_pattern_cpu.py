@@ -1,8 +1,8 @@
-"""solv compares the caller's pattern with the one its context holds.  A pattern
-that the library refuses leaves the context without any, so neither that pattern
-nor the one before it is the context's: the next call sets its structure first.
-The context is a stand-in that keeps the library's rules (values need a
-structure; a refused structure drops the one before)."""
+"""solv compares the caller's pattern with the one its context holds.  A structure
+that the library fails to build (out of memory) leaves the context without any, so
+neither that pattern nor the one before it is the context's: the next call sets its
+structure first.  The context is a stand-in that keeps the library's rules (values
+need a structure; one that fails drops the one before)."""
 import numpy as np
 import pytest
 
@@ -16,8 +16,8 @@ class _Held:
     def set_structure(self, ia, ja):
         self.calls.append("structure")
         self.pattern = None
-        if ja.size and ja.max() > len(ia) - 1:
-            raise _lib.ElasticError(_lib.BAD_ARG, "column outside the system")
+        if ja.size and ja.max() > 4:
+            raise _lib.ElasticError(_lib.OOM, "device memory")
         self.pattern = (ia.copy(), ja.copy())
 
     def set_values(self, ad, al):
@@ -30,7 +30,7 @@ class _Held:
         return np.array(b), {}
 
 
-PATTERNS = {"first": [1, 1, 2], "second": [1, 2, 3], "refused": [1, 2, 9], "longer": [1, 1, 2, 3]}
+PATTERNS = {"first": [1, 1, 2], "second": [1, 2, 3], "failing": [1, 2, 9], "longer": [1, 1, 2, 3]}
 
 
 def _call(name):
@@ -45,12 +45,12 @@ def _call(name):
 
 @pytest.mark.parametrize("before", ["first", "longer"])
 @pytest.mark.parametrize("after", ["first", "second", "longer"])
-def test_a_refused_pattern_does_not_stand_in_the_way(monkeypatch, before, after):
+def test_a_structure_that_fails_does_not_stand_in_the_way(monkeypatch, before, after):
     c = _Held()
     monkeypatch.setattr(solver, "_default_ctx", c)
     _call(before)
     with pytest.raises(_lib.ElasticError):
-        _call("refused")
+        _call("failing")
     ja = _call(after)
     assert np.array_equal(c.used[0], ja) and len(c.used[1]) == len(ja)
 

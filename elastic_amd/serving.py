@@ -119,16 +119,34 @@ def request_policy(ctx) -> tuple[int, int]:
     return FP64, 2
 
 
+# Systems of up to this many tiles iterate on the chip; a tile holds at most
+# CHIP_TILE_NODES nodes and 1024 node blocks
+CHIP_TILES, CHIP_TILE_NODES, CHIP_TILE_BLOCKS = 1024, 127, 1024
+
+
+def chip_bytes(nnode: int, ndf: int, per_node_lower: float) -> int:
+    """Device bytes of the words that the workgroups of a solve on the chip exchange
+    (0 where no layout of the system fits): slots, three rounds of a vector, two of
+    the tiles' external partials, of which there are up to one per node in 2-D and
+    three in 3-D."""
+    if nnode > CHIP_TILES * CHIP_TILE_NODES or nnode * per_node_lower > CHIP_TILES * CHIP_TILE_BLOCKS:
+        return 0
+    partials = nnode * (3 if ndf == 3 else 1.05)
+    return int(8 * (8 * (4 * 2 * 256 + 32) + ndf * (3 * nnode + 2 * partials)))
+
+
 def footprint_bytes(mesh) -> int:
     """Device bytes a prepared request holds, from its mesh alone (admission
     happens before anything is allocated): CSRC (ia, ja, al, ad), the blocked
-    FP64 and FP32 planes, layout words and merge lists, the external partials
-    and 9 FP64 vectors, with nad estimated from the element type's stencil."""
+    FP64 and FP32 planes, layout words and merge lists, the external partials,
+    9 FP64 vectors and the words of a solve on the chip, with nad estimated from
+    the element type's stencil."""
     ndf = mesh.ndf
     neq = int(mesh.nnode) * ndf
     per_node_lower = {3: 3.5, 4: 4.5, 6: 7.5, 8: 13.5}.get(mesh.nen, 13.5)  # lower neighbours
     nad = int(neq * (per_node_lower * ndf + 1))
-    return int(4 * neq + 12 * nad + 12 * nad + nad // 2 + 16 * neq + 9 * 8 * neq + 64 * 1024 * 8)
+    return int(4 * neq + 12 * nad + 12 * nad + nad // 2 + 16 * neq + 9 * 8 * neq + 64 * 1024 * 8
+               + chip_bytes(int(mesh.nnode), ndf, per_node_lower))
 
 
 @dataclass

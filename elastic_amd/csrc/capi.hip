@@ -601,8 +601,8 @@ int elastic_get_option(elastic_ctx* x, const char* name, int64_t* value) {
   else if (n == "time_products") *value = c->time_stride;
   else if (n == "tile_blocks") *value = effective_tile_blocks(c, c->layout_nb > 1 ? c->layout_nb : 3);
   else if (n == "tile_nnz") *value = c->tile_nnz;
-  else if (n == "lanes64") *value = c->lanes[0];
-  else if (n == "lanes32") *value = c->lanes[1];
+  else if (n == "lanes64") *value = tile_lanes(c, 0);
+  else if (n == "lanes32") *value = tile_lanes(c, 1);
   else if (n == "tune_tiles") *value = c->tune_tiles ? 1 : 0;
   else if (n == "layout_nb") *value = c->gather ? 0 : c->layout_nb;
   else if (n == "node_order") *value = c->blk.d2r ? 1 : 0;

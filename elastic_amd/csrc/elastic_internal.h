@@ -194,9 +194,10 @@ constexpr int kRedBlocks = 1024;  // fixed reduction grid (deterministic sums)
 // size on hex8 100^3); smaller systems and 2-dof nodes keep 512 (more tiles,
 // so more workgroups in flight; the batch's 2-D product holds 2 blocks per
 // lane).  3-dof systems of more than 512 tiles of 512 blocks take 1,024 too:
-// a resident solve then holds two tiles per CU instead of four smaller ones
-// (hex8 30^3, FP64: 9.7 against 12.4 us per iteration; with launches 26.0
-// against 24.7).
+// a resident solve then holds two tiles per CU instead of four smaller ones, and
+// BiCGSTAB, which holds no more than two, fits (hex8 30^3, FP64: PCG 9.2 against
+// 10.0 us per iteration, BiCGSTAB 21.6 against 54.3; PCG with launches 25.6 against
+// 24.5).
 constexpr int kTileBlocks3 = 1024, kTileBlocks2 = 512;
 constexpr int64_t kSmallTileBlocks = 512 * 512;
 constexpr int kLargeTileNodes = 32768;
@@ -209,9 +210,9 @@ struct Context {
   int64_t nad = 0;
   int tile_nnz = 2048;
   int tile_blocks = 0;         // node blocks per tile; 0: by node size (kTileBlocks3/2)
-  // lanes per tile of the node-blocked product (256 or 512), FP64 [0] and
-  // FP32-value [1] operators
-  int lanes[2] = {256, 256};
+  // lanes per tile of the node-blocked product (256 or 512; 0: tile_lanes
+  // decides), FP64 [0] and FP32-value [1] operators
+  int lanes[2] = {0, 0};
   bool tune_tiles = true;      // elastic_autotune also tries tile sizes (else lanes only)
   int layout_nb = 1;           // 1: scalar tiles; 2 or 3: node-blocked tiles
   bool accum32 = false;        // FP32 operator: FP32 staging and sums (else FP64)
@@ -448,6 +449,21 @@ hipError_t gmres_resident_launch(Context* c, const double* bm, double* basis, do
 size_t resident_words(Context* c);
 // the layout has such words, and the context's solves may use them
 inline bool resident_on(const Context* c) { return c->resident && !c->res_off && c->res_x; }
+// Lanes per tile of the launched FP64 (0) or FP32-value (1) product, until the caller
+// or the autotuner sets them: 512 for the tiles of more than 512 blocks that 3-dof
+// systems of less than kLargeTileNodes nodes take for the chip (kSmallTileBlocks), of
+// which there are 1.1 to 1.5 per CU: with 256 a CU has half the wavefronts that tiles
+// of 512 blocks give it.  us per step or iteration of hex8 28^3 / 30^3 / 31^3, tiles of
+// 512 blocks, of 1,024 with 256 lanes and with 512: mixed GMRES 54.6 55.2 54.8 / 57.1
+// 58.0 57.1 / 58.0 59.0 57.7, mixed BiCGSTAB 65.2 66.7 65.8 / 63.8 65.8 64.5 / 63.9 65.9
+// 63.6, FP64 GMRES 55.9 57.1 56.9 / 58.9 60.0 59.8 / 59.7 61.1 60.3.  Larger systems gain
+// nothing from 512: PCG on 33^3 (456 tiles) 27.1 and 27.6, tet4 33^3 x 6 (301) 24.3 and
+// 24.6.
+inline int tile_lanes(const Context* c, int op32) {
+  if (c->lanes[op32] > 0) return c->lanes[op32];
+  return c->layout_nb == 3 && c->blk.nblk_max > kTileBlocks2 && c->neq / 3 < kLargeTileNodes ? 512
+                                                                                             : 256;
+}
 hipError_t pcg_resident_launch(Context* c, const PcgVecs& V, bool fp32_operator, int maxit,
                                double* dslots, int tpw, float* p32, float* r32, float* m32,
                                float* dx32);

@@ -180,7 +180,7 @@ void launch_spmv(Context* c, bool fp32, const double* x, double* y, double* epar
                  const float* dx) {
   hipStream_t s = c->stream;
   const DevBlocks& b = c->blk;
-  const int l32 = c->lanes[1], l64 = c->lanes[0];
+  const int l32 = tile_lanes(c, 1), l64 = tile_lanes(c, 0);
   if (c->layout_nb == 3) {
     if (fp32 && c->accum32) spmv_blocks_launch<float, float, 3>(b, b.v32, b.d32, x, y, epart, s, skip, dot, y32 ? 1 : 0, x32, l32);
     else if (fp32) spmv_blocks_launch<float, double, 3>(b, b.v32, b.d32, x, y, epart, s, skip, dot, 0, nullptr, l32);

@@ -253,7 +253,8 @@ int elastic_layout_info(elastic_ctx* ctx, int64_t* info4);
  * effect at the next elastic_set_structure. */
 int elastic_set_tile_nnz(elastic_ctx* ctx, int32_t tile_nnz);
 /* Tile size of the node-blocked layout (node blocks per tile, 32..1024; by
- * default 1024 for 3-dof systems of at least 32,768 nodes, else 512);
+ * default 1024 for 3-dof systems of at least 32,768 nodes or more than 262,144
+ * node blocks, else 512);
  * takes effect at the next elastic_set_structure. */
 int elastic_set_tile_blocks(elastic_ctx* ctx, int32_t tile_blocks);
 /* Tuning knobs (no counterpart in the reference): "tile_blocks" /
@@ -264,7 +265,9 @@ int elastic_set_tile_blocks(elastic_ctx* ctx, int32_t tile_blocks);
  * FP64; until set, 1 for PCG on 3-dof systems of at least 32,768 nodes,
  * else 0),
  * "lanes64" / "lanes32" (256 or 512 lanes per tile of the node-blocked FP64 /
- * FP32-value product, 4 or 2 blocks per lane; default 256), "tune_tiles"
+ * FP32-value product, 4 or 2 blocks per lane; until set, 512 for tiles of more
+ * than 512 blocks of 3-dof systems of less than 32,768 nodes, else 256),
+ * "tune_tiles"
  * (0: elastic_autotune keeps the tile size),
  * "check_every" (iterations between convergence polls),
  * "batch_precond" (2: the context's batched solves use Jacobi, the default;

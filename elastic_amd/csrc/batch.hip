@@ -826,6 +826,11 @@ static int resident_variant(const Context* c, bool mixed, bool v32, int ncu) {
   return (mixed ? 2 : 0) + (b.nb == 3 ? 1 : 0);
 }
 
+bool batch_holds(const Context* c, bool mixed) {
+  const bool v32 = mixed && c->accum32 && c->batch_precond != ELASTIC_PRECOND_BDIAG3;
+  return c->layout_nb > 1 && resident_variant(c, mixed, v32, c->ncu) >= 0;
+}
+
 // every word of an instance says that it has not arrived (resident.h); later
 // steps find the words as the step before left them
 __global__ __launch_bounds__(256) void k_bt_res_empty(const BInst* __restrict__ insts, int slot) {

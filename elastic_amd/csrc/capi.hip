@@ -507,10 +507,13 @@ int solve_resident(elastic_ctx* x, int solver, int precond, int precision, doubl
                    int ngram, elastic_stats* st);
 }
 
-// Average device time of the products of a short resident PCG run of
-// `iters` iterations (b = ones; the caller's b is kept and put back; x is
-// overwritten), sampled with HIP events on every iteration.
-static int time_in_solve(elastic_ctx* x, int precision, int iters, double* ms) {
+// A short PCG run of `iters` iterations on the resident values (b = ones; the
+// caller's b is kept and put back; x is overwritten), by launches or, where the
+// layout is held, on the chip: *product, the average device time of its products
+// (HIP events around every one), and *iteration, the device time per iteration; in
+// ms.
+static int time_in_solve(elastic_ctx* x, int precision, int iters, bool on_chip, double* product,
+                         double* iteration) {
   Context* c = &x->c;
   const size_t nb = sizeof(double) * (size_t)c->neq;
   ELASTIC_HIP_CHECK(c, hipMemcpyAsync(c->v64[VW], c->v64[VB], nb, hipMemcpyDeviceToDevice, c->stream));
@@ -519,15 +522,16 @@ static int time_in_solve(elastic_ctx* x, int precision, int iters, double* ms) {
   const int stride = c->time_stride;
   const double tsum = c->tprod_ms;
   const int64_t tn = c->tprod_n;
-  c->time_stride = 1;
+  c->time_stride = on_chip ? 0 : 1;
   c->tprod_ms = 0.0;
   c->tprod_n = 0;
   const bool resident = c->resident;
-  c->resident = false;  // the candidates are products of a launch each
+  c->resident = resident && on_chip;
   elastic_stats st;
   int rc = solve_resident(x, ELASTIC_SOLVER_PCG, ELASTIC_PRECOND_DIAG, precision, 1e-300, iters,
                           50, &st);
-  *ms = c->tprod_n ? c->tprod_ms / (double)c->tprod_n : 1e300;
+  *product = c->tprod_n ? c->tprod_ms / (double)c->tprod_n : 1e300;
+  *iteration = st.iters > 0 ? st.t_device_ms / (double)st.iters : 1e300;
   c->resident = resident;
   c->time_stride = stride;
   c->tprod_ms = tsum;
@@ -539,7 +543,12 @@ static int time_in_solve(elastic_ctx* x, int precision, int iters, double* ms) {
 
 // Autotuner: for each candidate layout (node-blocked: tile size x lanes per
 // tile; scalar rows: tile size) runs a short resident PCG of the given
-// precision and keeps the candidate whose products are fastest on average.
+// precision.  Candidates that the chip holds come first, the one with the fastest
+// iteration there, since that is what a solve runs; among the others the one
+// whose products are fastest on average.  A candidate that would lose a place on
+// the chip that the current layout has, of a solve or of a batch's instance, is
+// not taken.  The lanes, which only launched products use, are those of the
+// fastest product of the tile size.
 // The tile size is shared by both operators (one layout); the lanes are
 // kept per precision.  With the option "tune_tiles" = 0 only the lanes are
 // tuned.
@@ -551,7 +560,8 @@ int elastic_autotune(elastic_ctx* x, int32_t precision, int32_t reps, int32_t* b
   if (c->gather) return set_error(c, ELASTIC_BAD_ARG, "the gather product has no tiles to tune");
   hipSetDevice(c->device);
   const bool blocked = c->layout_nb > 1;
-  const int pi = precision == ELASTIC_MIXED ? 1 : 0;
+  const bool mixed = precision == ELASTIC_MIXED;
+  const int pi = mixed ? 1 : 0;
   auto current = [&]() { return blocked ? effective_tile_blocks(c, c->layout_nb) : c->tile_nnz; };
   // the current layout is timed first and a candidate replaces the best
   // only when faster by more than 2%: timing noise does not move the layout
@@ -563,21 +573,44 @@ int elastic_autotune(elastic_ctx* x, int32_t precision, int32_t reps, int32_t* b
   const int iters = std::max(16, (int)reps);
   const bool verbose = getenv("ELASTIC_VERBOSE") != nullptr;
   int bt = -1, bl = 256;
-  double tmin = 1e300;
+  double tmin = 1e300, product = 1e300;
+  bool held = false, in_batch = false;  // of the best; of the current layout's instances
   for (int v : tiles) {
     if (v != current()) {
       int rc = blocked ? relayout(x, v, c->tile_nnz) : relayout(x, c->tile_blocks, v);
       if (rc) return rc;
     }
+    int lanes_v = 256;
+    double ms_v = 1e300;
     for (int lanes : {256, 512}) {
       if (lanes == 512 && (!blocked || c->blk.nblk_max <= 256)) continue;
       c->lanes[pi] = lanes;
-      double ms = 0.0;
-      int rc = time_in_solve(x, precision, iters, &ms);
+      double ms = 0.0, unused;
+      int rc = time_in_solve(x, precision, iters, false, &ms, &unused);
       if (rc && rc != ELASTIC_MAXIT) return rc;
       if (verbose) fprintf(stderr, "elastic_autotune: tile %d lanes %d product %.4f ms\n", v, lanes, ms);
-      if (ms < 0.98 * tmin) tmin = ms, bt = v, bl = lanes;
+      if (ms < 0.98 * ms_v) ms_v = ms, lanes_v = lanes;
     }
+    bool held_v = false;
+    double t = ms_v;
+    if (tiles.size() > 1 && resident_on(c)) {
+      double ms = 1e300;
+      for (int k = 0; k < 5; ++k) {
+        double unused, one;
+        int rc = time_in_solve(x, precision, 2 * iters, true, &unused, &one);
+        if (rc && rc != ELASTIC_MAXIT) return rc;
+        held_v = c->res_tiles > 0;
+        if (!held_v) break;
+        ms = std::min(ms, one);
+      }
+      if (held_v) t = ms;
+      if (verbose && held_v) fprintf(stderr, "elastic_autotune: tile %d on the chip %.4f ms\n", v, t);
+    }
+    const bool batch_v = batch_holds(c, mixed);
+    if (v == tiles[0]) in_batch = batch_v;
+    const bool loses = (held && !held_v) || (in_batch && !batch_v);
+    if (!loses && (bt < 0 || (held_v && !held) || t < 0.98 * tmin))
+      tmin = t, bt = v, bl = lanes_v, held = held_v, product = ms_v;
   }
   c->lanes[pi] = bl;
   if (bt > 0 && bt != current()) {
@@ -585,7 +618,7 @@ int elastic_autotune(elastic_ctx* x, int32_t precision, int32_t reps, int32_t* b
     if (rc) return rc;
   }
   if (best) *best = current();
-  if (best_ms) *best_ms = tmin;
+  if (best_ms) *best_ms = product;
   return ELASTIC_OK;
 }
 
@@ -609,6 +642,8 @@ int elastic_get_option(elastic_ctx* x, const char* name, int64_t* value) {
   else if (n == "resident") *value = resident_on(c) ? 1 : 0;
   else if (n == "resident_looks") *value = c->resident_looks;
   else if (n == "resident_tiles") *value = c->res_tiles;
+  else if (n == "resident_batch")
+    *value = (batch_holds(c, false) ? 1 : 0) + (batch_holds(c, true) ? 2 : 0);
   else if (n == "resident_lost") *value = c->res_lost;
   else return set_error((Context*)c, ELASTIC_BAD_ARG, "unknown option " + n);
   return ELASTIC_OK;

@@ -449,6 +449,9 @@ hipError_t gmres_resident_launch(Context* c, const double* bm, double* basis, do
 size_t resident_words(Context* c);
 // the layout has such words, and the context's solves may use them
 inline bool resident_on(const Context* c) { return c->resident && !c->res_off && c->res_x; }
+// batch.hip: whether an instance of the context, as its options are, iterates on the
+// chip
+bool batch_holds(const Context* c, bool mixed);
 // Lanes per tile of the launched FP64 (0) or FP32-value (1) product, until the caller
 // or the autotuner sets them: 512 for the tiles of more than 512 blocks that 3-dof
 // systems of less than kLargeTileNodes nodes take for the chip (kSmallTileBlocks), of

@@ -187,7 +187,8 @@ class Server:
     request.
     autotune True: the first request of each size class (node block size,
     precision and the bit length of neq) runs elastic_autotune before its
-    solve; later requests of the class take the tile size and lanes it chose.
+    solve; later requests of the class take the lanes it chose, and the tile size
+    unless that would take them off the chip.
     """
 
     def __init__(self, device: int = 0, max_slots: int = 64, iters_per_step: int = 16,
@@ -222,8 +223,14 @@ class Server:
             self.tuned[key] = (tile, ctx.get_option(lanes_opt))
             return
         tile, lanes = hit
-        if ctx.get_option(tile_opt) != tile:
+        own = ctx.get_option(tile_opt)
+        if own != tile:
+            # (not if this request, larger than the tuned one, would lose the chip)
+            names = ("resident", "resident_batch")
+            chip = [ctx.get_option(o) for o in names]
             ctx.set_option(tile_opt, tile)
+            if any(had & ~ctx.get_option(o) for had, o in zip(chip, names)):
+                ctx.set_option(tile_opt, own)
         ctx.set_option(lanes_opt, lanes)
 
     def run(self, requests: list[Request], realtime: bool = True) -> dict:

@@ -308,10 +308,13 @@ int elastic_product_timing(elastic_ctx* ctx, double* avg_ms, int64_t* count, int
  * overwritten) for each candidate layout -- node-blocked: 256, 512, 768 and
  * 1024 blocks per tile, each with 256 and 512 lanes per tile (4 or 2 blocks
  * per lane); scalar rows: 1024 to 3840 nonzeros per tile -- and keeps the
- * candidate whose products are fastest on average (HIP events around every
- * product of the run).  The tile size is shared by both operators; the lanes
+ * candidate that iterates fastest on the chip (option "resident") or, where none
+ * is held there, whose products are fastest on average (HIP events around every
+ * product of the run).  A tile size that would take a place on the chip from the
+ * context's solves or from its instances in a batch is not chosen.  The tile size is shared by both operators; the lanes
  * are kept for the given precision.  With the option "tune_tiles" = 0 only
- * the lanes are tuned.  Returns the tile size and the product time.  Not
+ * the lanes are tuned.  Returns the tile size and the time of its
+ * launched product.  Not
  * while the context is in a batch. */
 int elastic_autotune(elastic_ctx* ctx, int32_t precision, int32_t reps, int32_t* best,
                      double* best_ms);
@@ -323,6 +326,8 @@ int elastic_autotune(elastic_ctx* ctx, int32_t precision, int32_t reps, int32_t*
  * one of FP64 and FP32 sums fits) and they may be used; "resident_tiles": tiles
  * per workgroup with which the last solve, or the last instance that left a batch,
  * iterated on the chip (0: by launches, or started over with them);
+ * "resident_batch": whether a batch would hold an instance of it there, in FP64 (+1)
+ * and MIXED (+2);
  * "resident_lost": solves and instances of this context that started over. */
 int elastic_get_option(elastic_ctx* ctx, const char* name, int64_t* value);
 

@@ -119,8 +119,9 @@ static hipError_t res_run(Context* c, const PcgVecs& V, const TV* vals, const TV
                           res_tile_lds(sizeof(T), b.nb, b.ncols_max, b.nblk_max, c->res_merge,
                                        res_one_buffer(sizeof(T), b.nblk_max, tpw))};
   resident_clear(c, sizeof(T));
-  return b.nb == 3 ? res_dispatch<TV, T, VT, XT, 3>(c, g, tpw)
-                   : res_dispatch<TV, T, VT, XT, 2>(c, g, tpw);
+  if constexpr (sizeof(T) == 8)  // (no plan for FP32 sums in 2-D)
+    if (b.nb == 2) return res_dispatch<TV, T, VT, XT, 2>(c, g, tpw);
+  return res_dispatch<TV, T, VT, XT, 3>(c, g, tpw);
 }
 
 int pcg_resident_plan(Context* c, bool fp32_operator, bool bdiag, bool v32) {

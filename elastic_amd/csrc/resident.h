@@ -9,6 +9,12 @@
 // exchanges take 2.1 and 2.3, the product 1.8; with four tiles of 1,024 blocks per CU
 // and FP64 sums (hex8 43^3, 19.6 us) they take 4.2, 5 and 7.5.
 //
+// Where 1,024 lanes share a CU a lane has 128 registers: five of the kernels keep some
+// values in scratch then (bytes per lane in tests/test_resident_resources.py).  Only
+// PCG with FP64 sums on four tiles of up to 1,024 blocks re-reads matrix values, 7 of a
+// lane's 36 in each pass of the product; the others one or two doubles per iteration
+// or what a batch needs between instances.
+//
 // Everything that crosses workgroups goes through relaxed agent-scope atomics
 // (write-through stores, loads that do not take a line another XCD may hold
 // newer), never through fences: a device-scope fence writes back and

@@ -69,7 +69,7 @@ __device__ __forceinline__ void res_pcg(const ResPcg<TV, T, VT, XT>& g, int G, i
   if constexpr (STEP) asm volatile("" : "+v"(lane));
   const int grp = __builtin_amdgcn_readfirstlane(lane >> 8);  // uniform: scalar registers
   SolveScalars* sc = g.sc;
-  if (lane == 0) sh.bad = 0;
+  if (lane == 0) sh.bad = sh.late = 0;
   typedef ResTile<TV, T, NB, PER, TPW == 4, res_one<T, PER, TPW>()> Tile;
   constexpr bool MEM = res_vec_mem<T, PER, TPW>();
   const int tid = Tile::lane_of_tile(lane);
@@ -204,9 +204,12 @@ __device__ __forceinline__ void res_pcg(const ResPcg<TV, T, VT, XT>& g, int G, i
         apr += (double)pv * (double)rv[c];
       }
     }
+    // (told as sh.bad behind the barrier only: a wavefront that still reads that for
+    // the exchange would leave alone, its barriers meeting those of a batch's next
+    // instance)
     if (!t.ext_each(zc, e0, E, g.limit,
                     [&](int e, double ze) { xe[e] = (T)fma(beta, (double)xe[e], ze); }))
-      sh.bad = 1;
+      sh.late = 1;
     ++iter;
     ++k3;
     const double rn = sqrt(fabs(di)), conv = sh.keep[0];
@@ -223,7 +226,10 @@ __device__ __forceinline__ void res_pcg(const ResPcg<TV, T, VT, XT>& g, int G, i
       state = 3;
     }
     __syncthreads();  // p is staged, and everyone has used the last r.z
-    if (lane == 0) sh.keep[2] = di;
+    if (lane == 0) {
+      sh.keep[2] = di;
+      if (sh.late) sh.bad = 1;
+    }
     if (state) break;
   }
   __syncthreads();

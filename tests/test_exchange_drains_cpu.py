@@ -70,3 +70,18 @@ def test_every_word_is_visibly_empty_before_its_next_round(name, rounds):
 def test_the_check_finds_a_missing_drain():
     assert _undrained("DXXDXX") is None
     assert _undrained("DXXX") == 0 and _undrained("XXDXXX") == 2
+
+
+def test_a_lost_word_is_told_behind_a_barrier():
+    """In the PCG kernel, whose workgroups go on to a batch's next instance, the
+    flag that a wait ran out changes only where every wavefront reads the same: in
+    an exchange before its last barrier, or behind a barrier that follows it.  (Set
+    earlier, a slow wavefront would see it as the exchange's and leave the loop alone,
+    one barrier off from the others.)"""
+    text = re.sub(r"//[^\n]*", "", open(os.path.join(CSRC, "pcg_resident.h")).read())
+    body, _ = _block(text, text.index("while (true)"))
+    marks = re.findall(r"res_exchange<|__syncthreads\(\)|sh\.bad = 1", body)
+    assert marks.count("sh.bad = 1") == 1
+    for k, m in enumerate(marks):
+        if m == "sh.bad = 1":
+            assert marks[k - 1] == "__syncthreads()", marks

@@ -28,9 +28,12 @@
 // after the other, each system with exchange words of its own.  Per batch, lists
 // against resident: 16 plane sections of up to 160^2 elements 66.4 and 29.2 ms,
 // 8 hex8 12^3 8.0 and 3.3, 6 hex8 33^3 mixed 50.8 and 31.8, 64 plane requests of up
-// to 512^2 (lists and chip together) 2,537 and 2,458.  Where every instance is large
-// (16 of 390 to 1,030 tiles, one or two on the chip at a time) the lists were 7%
-// faster, 418 against 449; an instance may not look at the others, so it stays.
+// to 512^2 (lists and chip together) 2,537 and 2,458, 16 of 224^2 to 360^2 (397 to
+// 1,024 tiles) 424 and 370.  The lists are faster where a dozen or more instances of
+// the same 513 to 720 tiles leave half of the CUs idle, one at a time (16 quad4 256^2
+// 191 and 243, 32 tria3 258^2 620 and 896; but 2 quad4 256^2 60 and 33).  An instance may
+// not look at the others, whose bits would depend on the mix, and sending those sizes
+// to the lists costs mixed sizes more (370 to 431) than it gives.
 #include <algorithm>
 #include <chrono>
 #include <cmath>

@@ -69,7 +69,10 @@ __device__ __forceinline__ void res_pcg(const ResPcg<TV, T, VT, XT>& g, int G, i
   if constexpr (STEP) asm volatile("" : "+v"(lane));
   const int grp = __builtin_amdgcn_readfirstlane(lane >> 8);  // uniform: scalar registers
   SolveScalars* sc = g.sc;
-  if (lane == 0) sh.bad = sh.late = 0;
+  if (lane == 0) {
+    sh.bad = 0;
+    if constexpr (STEP) sh.late = 0;
+  }
   typedef ResTile<TV, T, NB, PER, TPW == 4, res_one<T, PER, TPW>()> Tile;
   constexpr bool MEM = res_vec_mem<T, PER, TPW>();
   const int tid = Tile::lane_of_tile(lane);
@@ -204,12 +207,15 @@ __device__ __forceinline__ void res_pcg(const ResPcg<TV, T, VT, XT>& g, int G, i
         apr += (double)pv * (double)rv[c];
       }
     }
-    // (told as sh.bad behind the barrier only: a wavefront that still reads that for
-    // the exchange would leave alone, its barriers meeting those of a batch's next
-    // instance)
+    // (in a batch told as sh.bad behind the barrier only: a wavefront that still reads
+    // that for the exchange would leave alone, its barriers meeting those of the next
+    // instance.  A single solve ends there, lost; the flag's read behind the barrier
+    // would cost it 0.3 to 0.7%)
     if (!t.ext_each(zc, e0, E, g.limit,
-                    [&](int e, double ze) { xe[e] = (T)fma(beta, (double)xe[e], ze); }))
-      sh.late = 1;
+                    [&](int e, double ze) { xe[e] = (T)fma(beta, (double)xe[e], ze); })) {
+      if constexpr (STEP) sh.late = 1;
+      else sh.bad = 1;
+    }
     ++iter;
     ++k3;
     const double rn = sqrt(fabs(di)), conv = sh.keep[0];
@@ -228,7 +234,8 @@ __device__ __forceinline__ void res_pcg(const ResPcg<TV, T, VT, XT>& g, int G, i
     __syncthreads();  // p is staged, and everyone has used the last r.z
     if (lane == 0) {
       sh.keep[2] = di;
-      if (sh.late) sh.bad = 1;
+      if constexpr (STEP)
+        if (sh.late) sh.bad = 1;
     }
     if (state) break;
   }

@@ -110,7 +110,7 @@ struct ResShared {
   double sum[2][4];              // wavefront sums over the workgroups
   double keep[4];                // scalars of the method
   int bad;                       // a wait ran out: every workgroup gives up
-  int late;                      // the same, outside of an exchange (pcg_resident.h)
+  int late;                      // the same, outside of an exchange, in a batch's step (pcg_resident.h)
 };
 
 // v[k] = its sum over all lanes (this one tid) of the system's workgroups (this
